@@ -30,6 +30,14 @@ constexpr size_t teno_lin_off(size_t b, int Mp, int i, uint32_t cl, int FQ, int 
 // face's node 0 is the cell node hi of the edge (lo, hi) in bits 24 + 2 l)
 constexpr int face_flip_shift(int l) { return l == 0 ? 30 : (l == 1 ? 31 : 19); }
 
+// Bits of a face-list entry's meta word: the face's slot in its side-0 and
+// side-1 cells, the boundary flag and the boundary condition's index.
+constexpr uint32_t kFaceSlot1Shift = 2, kFaceBoundary = 1u << 4, kFaceBcShift = 5;
+// Bits of a cell's face-sum word: rank r -> slot (2 bits each, from bit 0),
+// the number of contributing slots (bits 8-10), per slot the cell's side of
+// the face (bit 11 + slot) and whether it is a boundary face (bit 15 + slot).
+constexpr uint32_t kSumCountShift = 8, kSumSideShift = 11, kSumBoundaryShift = 15;
+
 struct Physics {
     double gamma, R, cp, cv, p_min, p_max;
     // Navier-Stokes: viscous != 0 adds the viscous fluxes; Sutherland law
@@ -59,6 +67,17 @@ struct Geom {
     const double* dcy;    //        midpoint on boundaries (viscous runs only)
     const double* mfx;    // [S][N] centroid to face midpoint (viscous runs only)
     const double* mfy;
+    // face lists per 64-cell block (flux kernel)
+    const uint32_t* face_off;
+    const uint32_t* face_c0;
+    const uint32_t* face_c1;
+    const uint16_t* face_meta;
+    const double* face_nx;
+    const double* face_ny;
+    const double* face_area;
+    const uint32_t* cell_faces;  // [N]
+    const uint32_t* cell_sum;    // [N]
+    uint32_t face_max[3];        // most list entries of a 64-, 128- and 256-cell flux block
 };
 
 namespace ind {
@@ -150,6 +169,7 @@ struct StageArgs {
     // is the cell mean (a zero-gradient ghost cell) instead of the face state
     int32_t corrected;
     int32_t pp;           // 1: positivity-preserving flux limiter (stage updates)
+    int32_t parts;        // face sums taken: 1 interior, 2 boundary (kRhsOnly), 3 both
     const double* Uin;    // stage input state (gathered), [N][4]
     const double* Un;     // step start state
     double* Uout;
@@ -199,12 +219,8 @@ struct Tune {
 // evaluating the network again (later stages of a step)
 hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs, uint8_t* decisions,
                       const Physics& ph, int occ, int gate_reuse, hipStream_t stream);
-// bs: cells (threads) per block
+// bs: cells per block
 hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream);
-// kRhsOnly residual over the faces `parts` selects: 1 interior, 2 boundary,
-// 3 both (the full residual, flux_update)
-hipError_t rhs_parts(const Geom& g, const StageArgs& a, const Physics& ph, int parts, uint32_t bs,
-                     hipStream_t stream);
 // spectral radii: lam_cell per cell and, per bs-cell block, the bit pattern
 // of the block's largest radius in lam_blk (NaN radii are ignored)
 hipError_t spectral_radius(const Geom& g, const double* Un, const double* prims, const Physics& ph,
@@ -220,7 +236,8 @@ hipError_t viscous_grad(const Geom& g, const double* U, const Physics& ph, doubl
 // Ensemble launchers: `cases` is a device array of n_cases descriptors whose
 // blk_* offsets are prefix sums (flux and spectral blocks of bs cells, TENO
 // blocks of 64); every case has the same K, M, face points, tile-position
-// width (small = 8-bit) and Riemann solver.
+// width (small = 8-bit) and Riemann solver. face_max: the largest number of
+// face-list entries of a flux block in any case.
 // gated: some case runs the learned gate (the block stages the network in LDS);
 // split: every case's gate runs split (Teno::blk_mixed set), as teno_faces
 // derived: plain pass with every case's face basis derived (Teno::derived)
@@ -228,7 +245,7 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
                       bool small, bool gated, int occ, int gate_reuse, bool split, bool derived, const Physics& ph,
                       hipStream_t stream);
 hipError_t flux_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const BatchStage& st, int riemann,
-                      const Physics& ph, uint32_t bs, hipStream_t stream);
+                      const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream);
 hipError_t spectral_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const Physics& ph, uint32_t bs,
                           hipStream_t stream);
 hipError_t finalize_batch(const CaseBufs* cases, int n_cases, double cfl, double fixed_dt, int64_t hist_cap,
@@ -258,8 +275,8 @@ struct PersistentStep {
     long long spin_ticks;  // longest wait at a barrier, device wall-clock ticks
 };
 hipError_t ensemble_step(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
-                         const PersistentStep& ps, int riemann, bool teno, const Physics& ph, hipStream_t stream,
-                         int* grid_out);
+                         const PersistentStep& ps, int riemann, bool teno, uint32_t face_max, const Physics& ph,
+                         hipStream_t stream, int* grid_out);
 hipError_t probe_math(const double* x, const double* y, double* out, int n, int which, hipStream_t stream);
 
 // Point-wise operators (operators.hip).

@@ -70,6 +70,12 @@ uint64_t Ensemble::n_cells() const {
     return n;
 }
 
+uint32_t Ensemble::face_max(uint32_t bs) const {
+    uint32_t n = 0;
+    for (const auto& c : cases_) n = std::max(n, c->L_.face_max[bs == 64 ? 0 : (bs == 128 ? 1 : 2)]);
+    return n;
+}
+
 void Ensemble::upload_table() {
     std::vector<dev::CaseBufs> tab;
     tab.reserve(cases_.size());
@@ -169,7 +175,8 @@ void Ensemble::autotune() {
         upload_table();
         const float t = timed([&] {
             hip_ok(dev::spectral_batch(d_cases_, n, flux_blocks_, ph_, bs, stream_), "spectral_batch");
-            hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, stream_), "flux_batch");
+            hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
+                   "flux_batch");
         });
         if (t < bt) { bt = t; best.flux_block = bs; }
     }
@@ -260,7 +267,8 @@ void Ensemble::launch_step(bool prof) {
             mark(kStatTenoMs);
         }
         const dev::BatchStage st{op, teno_ ? 0 : 1, corrected, in, out, cfg_.positivity ? 1 : 0};
-        hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, stream_), "flux_batch");
+        hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
+                   "flux_batch");
         mark(kStatFluxMs);
     };
     if (cfg_.integrator == Integrator::SSPRK3) {
@@ -353,8 +361,8 @@ void Ensemble::launch_persistent(long long* clocks) {
     ps.cfl = cfg_.cfl;
     ps.fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
     ps.hist_cap = cases_[0]->dt_hist_cap_;
-    hip_ok(dev::ensemble_step(d_cases_, size(), teno_blocks_, flux_blocks_, ps, (int)cfg_.riemann, teno_, ph_, stream_,
-                              &persistent_grid_), "ensemble_step");
+    hip_ok(dev::ensemble_step(d_cases_, size(), teno_blocks_, flux_blocks_, ps, (int)cfg_.riemann, teno_,
+                              face_max(256), ph_, stream_, &persistent_grid_), "ensemble_step");
 }
 
 void Ensemble::finish(int64_t s0, int64_t n) {

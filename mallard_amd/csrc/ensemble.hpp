@@ -62,6 +62,7 @@ public:
 
 private:
     void upload_table();
+    uint32_t face_max(uint32_t bs) const;  // most face-list entries of a bs-cell flux block in any case
     void launch_step(bool prof);
     void launch_persistent(long long* clocks);
     void run_steps_profiled_persistent(int64_t n, double* stats);

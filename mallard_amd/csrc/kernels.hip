@@ -23,7 +23,6 @@ namespace {
 
 constexpr uint32_t kBoundaryBit = 1u << 3;
 
-
 struct D4 {
     double v[4];
 };
@@ -704,34 +703,31 @@ __global__ __launch_bounds__(256) void viscous_grad_kernel(Geom g, const double*
 }
 
 // Viscous flux through a face, in the face's orientation (unit normal n from
-// its side-0 cell L to R): G = (0, tau n, (u tau + k grad T) n). Face
+// its side-0 cell L, slot sL, to R, slot sR): G = (0, tau n, (u tau + k grad T) n). Face
 // gradients are the mean of the two cells' gradients with the directional
 // derivative along d = x_R - x_L replaced by (phi_R - phi_L) / |d|; the face
 // velocity is the mean of both cells' linear extrapolations to the face
 // midpoint. On a boundary face the cell's gradient is corrected toward the
 // boundary value along the centroid-to-midpoint vector. All of it is exact
-// for linear fields, and both cells of a face evaluate the same operations on
-// the same values, so they agree bit for bit.
-__device__ inline void viscous_face(const Physics& ph, const Geom& g, const StageArgs& a, size_t o, uint32_t c,
-                                    uint32_t inf, bool bnd, uint32_t side, double n0, double n1, double* G) {
+// for linear fields.
+__device__ inline void viscous_face(const Physics& ph, const Geom& g, const StageArgs& a, uint32_t L, uint32_t sL,
+                                    uint32_t R, uint32_t sR, bool bnd, uint32_t bc, double n0, double n1, double* G) {
     G[0] = 0.0; G[1] = 0.0; G[2] = 0.0; G[3] = 0.0;
     int bt = -1;
     if (bnd) {
-        bt = g.bc[(inf >> 4) & 0xFu].type;
+        bt = g.bc[bc].type;
         if (bt == 0 || bt == 2) return;  // symmetry, slip wall: no viscous stress or heat flux
     }
-    const uint32_t L = (!bnd && side) ? (uint32_t)g.nb[o] : c;
+    const size_t oL = (size_t)sL * g.N + L;
     const D4 pL = ld4(a.vp, L);
     const double2* gL2 = reinterpret_cast<const double2*>(a.vg + 6 * (size_t)L);
     const double2 gL0 = gL2[0], gL1 = gL2[1], gL3 = gL2[2];
-    double dx = g.dcx[o], dy = g.dcy[o];
-    if (side) { dx = -dx; dy = -dy; }
+    const double dx = g.dcx[oL], dy = g.dcy[oL];
     const double il = 1.0 / sqrt(dx * dx + dy * dy);
     const double tx = dx * il, ty = dy * il;
     double gx[3], gy[3], uf, vf, mu;
     const double phL[3] = {pL.v[0], pL.v[1], pL.v[2]};
     if (!bnd) {
-        const uint32_t R = side ? c : (uint32_t)g.nb[o];
         const D4 pR = ld4(a.vp, R);
         const double2* gR2 = reinterpret_cast<const double2*>(a.vg + 6 * (size_t)R);
         const double2 gR0 = gR2[0], gR1 = gR2[1], gR3 = gR2[2];
@@ -745,9 +741,8 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
             gx[k] += corr * tx;
             gy[k] += corr * ty;
         }
-        // centroid-to-midpoint vectors of L and R (own slot and the neighbour's slot)
-        const size_t on = (size_t)(inf & 3u) * g.N + (uint32_t)g.nb[o];
-        const size_t oL = side ? on : o, oR = side ? o : on;
+        const size_t oR = (size_t)sR * g.N + R;
+        // centroid-to-midpoint vectors
         const double mLx = g.mfx[oL], mLy = g.mfy[oL], mRx = g.mfx[oR], mRy = g.mfy[oR];
         uf = 0.5 * ((pL.v[0] + (gL0.x * mLx + gL0.y * mLy)) + (pR.v[0] + (gR0.x * mRx + gR0.y * mRy)));
         vf = 0.5 * ((pL.v[1] + (gL1.x * mLx + gL1.y * mLy)) + (pR.v[1] + (gR1.x * mRx + gR1.y * mRy)));
@@ -757,7 +752,7 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
         gx[1] = gL1.x; gy[1] = gL1.y;
         gx[2] = gL3.x; gy[2] = gL3.y;
         double pf[3];
-        boundary_uvT(g.bc[(inf >> 4) & 0xFu], n0, n1, phL, pf);
+        boundary_uvT(g.bc[bc], n0, n1, phL, pf);
         if (bt != 1 && bt != 4) {  // a prescribed value: correct toward it
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -783,102 +778,75 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
 }
 
 // ------------------------------------------------------------ flux + update
-// One thread per cell: the residual of the cell in the canonical face order,
-// divided by the volume, then the stage's SSP-RK update (no atomics).
+// The fluxes of a block of cells, then the residual and the stage update of
+// each cell. A block of bs cells takes every face of its cells once (the
+// face lists of its 64-cell blocks), one face per thread and round, and leaves
+// area times flux in LDS; after a barrier one thread per cell sums its faces
+// in the canonical order, divides by the volume and applies the stage's
+// SSP-RK update (no atomics). A flux has the same bits for both cells of its
+// face, so the sums equal a serial run's in the one-thread order.
+// What bounds it: FP64 issue and the chain of divisions, square roots and
+// pows in one flux, then memory. Evaluating a face once per block instead of
+// once per cell takes 1.7 evaluations per cell instead of 3, and reads 58 B
+// of face lists instead of 96 B of slot arrays per cell. HLLC on a flow with
+// waves everywhere (rocprof, one thread per cell and its three faces before):
+// 8,388,608 cells 1,161 -> 895 us, 524,288 72.8 -> 51.9 us, 2,048 26.4 ->
+// 9 us; with the limiter, 73,006 cells 35 -> 16 us; viscous Roe, 99,700 cells
+// 22.8 -> 16 us. Holding the registers (105 for HLLC, 4 waves per SIMD) to 5
+// waves costs time: 8,388,608 cells 957 us, at 6 waves 1,110 us.
 // RS: Riemann solver (compile-time, so each instantiation carries one
-// solver's code and registers). Blocks follow the XCD-aware order of the
-// TENO kernel, so the neighbour face states a block gathers were written by
-// the same XCD.
-// PARTS: face sums taken, bit 0 interior faces, bit 1 boundary faces (3: the
-// whole residual; 1 or 2 only with kRhsOnly).
-// PP: the positivity-preserving flux limiter (pp_limit) on every face, for
-// the stage updates (not the residual-only operator, which has no dt).
-template <int RS, int PARTS = 3, bool PP = false>
-__device__ __forceinline__ void flux_cell(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t c) {
-    const uint32_t N = g.N;
-    if (c >= N) return;
-    const uint32_t Q = g.Q;
-    const uint32_t info0 = g.info[c];
-    const uint32_t code = (info0 >> 8) & 0xFFu, nact = (info0 >> 16) & 0x7u;
-    double r[4] = {0.0, 0.0, 0.0, 0.0};
-    D4 um{};
-    double vc = 0.0, pdt = 0.0;
+// solver's code and registers). PP: the positivity-preserving flux limiter
+// (pp_limit) on every face, for the stage updates (not the residual-only
+// operator, which has no dt). VISC: the viscous fluxes.
+template <int RS, bool PP, bool VISC>
+__device__ __forceinline__ void face_flux(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t e,
+                                          double* out) {
+    const uint32_t N = g.N, Q = g.Q;
+    const uint32_t meta = g.face_meta[e], c0 = g.face_c0[e], c1 = g.face_c1[e];
+    const uint32_t s0 = meta & 3u, s1 = (meta >> kFaceSlot1Shift) & 3u, bc = (meta >> kFaceBcShift) & 0xFu;
+    const bool bnd = (meta & kFaceBoundary) != 0;
+    const double n0 = g.face_nx[e], n1 = g.face_ny[e], ar = g.face_area[e];
+    double F[4] = {0.0, 0.0, 0.0, 0.0};
+    for (uint32_t q = 0; q < Q; ++q) {
+        D4 L, R;
+        if (a.fo) {
+            L = ld4(a.Uin, c0);
+            R = ld4(a.Uin, c1);
+        } else {
+            L = ld4(a.fs, (size_t)(s0 * Q + q) * N + c0);
+            // on a boundary (c1 = c0) the state an extrapolation boundary
+            // copies into its ghost: the face state itself
+            // (boundary_extrapolation.cpp:38-55), or in the corrected variant
+            // the cell mean
+            if (!bnd) R = ld4(a.fs, (size_t)(s1 * Q + q) * N + c1);
+            else R = a.corrected ? ld4(a.Uin, c0) : L;
+        }
+        double Ft[4];
+        point_flux(ph, g.bc, RS, a.corrected, bnd, bc, n0, n1, L.v, R.v, Ft);
+        const double wq = g.qw[q];
+#pragma unroll
+        for (int i = 0; i < 4; i++) F[i] += wq * Ft[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) F[i] *= 0.5;
     if constexpr (PP) {
-        um = ld4(a.Uin, c);
-        vc = g.volume[c];
-        pdt = *a.dt;
+        const D4 U0 = ld4(a.Uin, c0), U1 = ld4(a.Uin, c1);
+        const double Sd = (double)g.S, pdt = *a.dt;
+        pp_limit(ph, g.bc, bnd, bc, n0, n1, F, U0.v, Sd * pdt * ar / g.volume[c0], U1.v,
+                 Sd * pdt * ar / g.volume[c1]);
     }
-    for (uint32_t rk = 0; rk < nact; ++rk) {
-        const uint32_t l = (code >> (2 * rk)) & 3u;
-        const size_t o = (size_t)l * N + c;
-        const uint32_t inf = g.info[o];
-        const bool bnd = (inf & kBoundaryBit) != 0;
-        if constexpr (PARTS != 3) {
-            if (bnd ? !(PARTS & 2) : !(PARTS & 1)) continue;
-        }
-        const uint32_t side = (inf >> 2) & 1u;
-        const double n0 = g.nx[o], n1 = g.ny[o], ar = g.area[o];
-        double F[4] = {0.0, 0.0, 0.0, 0.0};
-        for (uint32_t q = 0; q < Q; ++q) {
-            D4 own, oth;
-            if (a.fo) {
-                own = ld4(a.Uin, c);
-            } else {
-                own = ld4(a.fs, (size_t)(l * Q + q) * N + c);
-            }
-            double Ft[4];
-            if (!bnd) {
-                const uint32_t nbc = (uint32_t)g.nb[o];
-                const uint32_t nbs = inf & 3u;
-                oth = a.fo ? ld4(a.Uin, nbc) : ld4(a.fs, (size_t)(nbs * Q + q) * N + nbc);
-                double L[4], R[4];  // selected by value (a selected pointer can put them in scratch)
+    if constexpr (VISC) {
+        double G[4];
+        viscous_face(ph, g, a, c0, s0, c1, s1, bnd, bc, n0, n1, G);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    L[i] = side ? oth.v[i] : own.v[i];
-                    R[i] = side ? own.v[i] : oth.v[i];
-                }
-                point_flux(ph, g.bc, RS, a.corrected, false, 0, n0, n1, L, R, Ft);
-            } else {
-                // the ghost state an extrapolation boundary copies: the face
-                // state itself (boundary_extrapolation.cpp:38-55), or in the
-                // corrected variant the cell mean
-                const D4 ghost = a.corrected ? ld4(a.Uin, c) : own;
-                point_flux(ph, g.bc, RS, a.corrected, true, (inf >> 4) & 0xFu, n0, n1, own.v, ghost.v, Ft);
-            }
-            const double wq = g.qw[q];
-#pragma unroll
-            for (int i = 0; i < 4; i++) F[i] += wq * Ft[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) F[i] *= 0.5;
-        if constexpr (PP) {
-            // in side order (side 0 first), so both cells of a face agree bit for bit
-            const uint32_t nbc = bnd ? c : (uint32_t)g.nb[o];
-            const D4 mo = bnd ? um : ld4(a.Uin, nbc);
-            const double vo = bnd ? vc : g.volume[nbc];
-            double U0[4], U1[4];  // selected by value: a selected pointer would put the means in scratch
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                U0[i] = side ? mo.v[i] : um.v[i];
-                U1[i] = side ? um.v[i] : mo.v[i];
-            }
-            const double V0 = side ? vo : vc, V1 = side ? vc : vo;
-            const double Sd = (double)g.S;
-            pp_limit(ph, g.bc, bnd, (inf >> 4) & 0xFu, n0, n1, F, U0, Sd * pdt * ar / V0, U1, Sd * pdt * ar / V1);
-        }
-        if (ph.viscous) {
-            double G[4];
-            viscous_face(ph, g, a, o, c, inf, bnd, side, n0, n1, G);
-#pragma unroll
-            for (int i = 1; i < 4; i++) F[i] -= G[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) r[i] += side ? ar * F[i] : -ar * F[i];
+        for (int i = 1; i < 4; i++) F[i] -= G[i];
     }
-    const double vol = g.volume[c];
 #pragma unroll
-    for (int i = 0; i < 4; i++) r[i] /= vol;
+    for (int i = 0; i < 4; i++) out[i] = ar * F[i];
+}
 
+// The stage's update of cell c with its residual r.
+__device__ __forceinline__ void stage_update(const StageArgs& a, const Physics& ph, uint32_t c, const double* r) {
     if (a.op == kRhsOnly) {
         st4(a.rhs, c, D4{{r[0], r[1], r[2], r[3]}});
         return;
@@ -950,46 +918,83 @@ __device__ __forceinline__ void flux_cell(const Geom& g, const StageArgs& a, con
     }
 }
 
-template <int RS, bool PP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PP ? 4 : 1, 8)))
-void flux_update_kernel(Geom g, StageArgs a, Physics ph, uint32_t blocks_per_xcd) {
-    const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    flux_cell<RS, 3, PP>(g, a, ph, lb * blockDim.x + threadIdx.x);
+// lb: flux block of bs cells; sf: LDS for 4 planes of its face-list entries
+template <int RS, bool PP, bool VISC>
+__device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t lb,
+                                           uint32_t bs, double* sf) {
+    const uint32_t N = g.N, first = lb * bs;
+    if (first >= N) return;  // whole block past the end (uniform)
+    const uint32_t last = N - first < bs ? N : first + bs;
+    const uint32_t f0 = g.face_off[first >> 6], nf = g.face_off[(last + 63u) >> 6] - f0;
+    for (uint32_t i = threadIdx.x; i < nf; i += blockDim.x) {
+        double F[4];
+        face_flux<RS, PP, VISC>(g, a, ph, f0 + i, F);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sf[k * nf + i] = F[k];
+    }
+    __syncthreads();
+    for (uint32_t c = first + threadIdx.x; c < last; c += blockDim.x) {
+        const uint32_t slots = g.cell_faces[c], sum = g.cell_sum[c];
+        const uint32_t base = g.face_off[c >> 6] - f0, count = (sum >> kSumCountShift) & 0x7u;
+        double r[4] = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t rk = 0; rk < count; ++rk) {
+            const uint32_t l = (sum >> (2 * rk)) & 3u;
+            if (!(a.parts & ((sum >> (kSumBoundaryShift + l)) & 1u ? 2 : 1))) continue;
+            const uint32_t i = base + ((slots >> (8 * l)) & 0xFFu);
+            const bool side = ((sum >> (kSumSideShift + l)) & 1u) != 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double f = sf[k * nf + i];
+                r[k] += side ? f : -f;
+            }
+        }
+        const double vol = g.volume[c];
+#pragma unroll
+        for (int k = 0; k < 4; k++) r[k] /= vol;
+        stage_update(a, ph, c, r);
+    }
 }
 
-// The residual restricted to the interior faces (PARTS = 1, the
-// reference's calc_rhs_interior) or to the boundary faces (PARTS = 2, its
-// calc_rhs_boundaries, i.e. every Boundary::apply), divided by the volume.
-template <int RS, int PARTS>
-__global__ __launch_bounds__(256) void rhs_parts_kernel(Geom g, StageArgs a, Physics ph, uint32_t blocks_per_xcd) {
+template <int RS, bool PP, bool VISC>
+__global__ __launch_bounds__(256) void flux_update_kernel(Geom g, StageArgs a, Physics ph, uint32_t bs,
+                                                          uint32_t blocks_per_xcd) {
+    extern __shared__ __align__(16) unsigned char flux_smem[];
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    flux_cell<RS, PARTS>(g, a, ph, lb * blockDim.x + threadIdx.x);
+    flux_block<RS, PP, VISC>(g, a, ph, lb, bs, reinterpret_cast<double*>(flux_smem));
 }
 
-// The flux + stage update of every case in one launch (blocks of blockDim.x
-// cells; the case table's block offsets count blocks of that size).
-template <int RS, bool PP>
-__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases, int n_cases,
-                                                         BatchStage st, uint32_t total, Physics ph,
-                                                         uint32_t blocks_per_xcd) {
-    const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    if (gb >= total) return;
-    const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+__device__ inline StageArgs case_stage(const CaseBufs& cs, int op, int riemann, int fo, int corrected, int in,
+                                       int out) {
     StageArgs a{};
-    a.op = st.op;
-    a.riemann = RS;
-    a.fo = st.fo;
-    a.corrected = st.corrected;
-    a.Uin = case_buf(cs, st.in);
+    a.op = op;
+    a.riemann = riemann;
+    a.fo = fo;
+    a.corrected = corrected;
+    a.parts = 3;
+    a.Uin = case_buf(cs, in);
     a.Un = cs.Un;
-    a.Uout = case_buf_w(cs, st.out);
+    a.Uout = case_buf_w(cs, out);
     a.W = cs.W;
     a.prims = cs.prims;
     a.h = cs.h;
     a.rhs = cs.rhs;
     a.fs = cs.fs;
     a.dt = cs.dt;
-    flux_cell<RS, 3, PP>(cs.g, a, ph, (gb - cs.blk_flux0) * blockDim.x + threadIdx.x);
+    return a;
+}
+
+// The flux + stage update of every case in one launch (blocks of bs cells;
+// the case table's block offsets count blocks of that size).
+template <int RS, bool PP>
+__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases, int n_cases,
+                                                         BatchStage st, uint32_t total, Physics ph, uint32_t bs,
+                                                         uint32_t blocks_per_xcd) {
+    extern __shared__ __align__(16) unsigned char flux_smem[];
+    const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
+    if (gb >= total) return;
+    const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+    const StageArgs a = case_stage(cs, st.op, RS, st.fo, st.corrected, st.in, st.out);
+    flux_block<RS, PP, false>(cs.g, a, ph, gb - cs.blk_flux0, bs, reinterpret_cast<double*>(flux_smem));
 }
 
 // ------------------------------------------------------------ dt
@@ -1228,21 +1233,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         stamp(3 + 2 * st);
         each(flux_total, [&](uint32_t gb) {
             const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
-            StageArgs a{};
-            a.op = ps.op[st];
-            a.riemann = RS;
-            a.fo = ps.fo;
-            a.corrected = ps.corrected;
-            a.Uin = case_buf(cs, ps.in[st]);
-            a.Un = cs.Un;
-            a.Uout = case_buf_w(cs, ps.out[st]);
-            a.W = cs.W;
-            a.prims = cs.prims;
-            a.h = cs.h;
-            a.rhs = cs.rhs;
-            a.fs = cs.fs;
-            a.dt = cs.dt;
-            flux_cell<RS>(cs.g, a, ph, (gb - cs.blk_flux0) * blockDim.x + threadIdx.x);
+            const StageArgs a = case_stage(cs, ps.op[st], RS, ps.fo, ps.corrected, ps.in[st], ps.out[st]);
+            flux_block<RS, false, false>(cs.g, a, ph, gb - cs.blk_flux0, blockDim.x,
+                                         reinterpret_cast<double*>(step_smem));
         });
         if (st + 1 < ps.n_stages || ps.clocks) grid_barrier(ps.bar, G, ps.spin_ticks);
         stamp(4 + 2 * st);
@@ -1488,15 +1481,34 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
     return hipGetLastError();
 }
 
+namespace {
+// Threads of a flux block of bs cells, whose faces number about 1.7 bs on
+// triangles and 2.2 bs on quads. While the whole mesh's faces fit the chip at
+// once (4 waves per SIMD hold 262,144 threads), a kernel lasts as long as one
+// thread's chain, and two threads per cell halve it: HLLC residual of 8,192
+// triangles 8.9 us against 14.1 us with one thread per cell, 131,072
+// triangles 16.3 against 18.2. On larger meshes the second half of the block
+// idles in the cell sums: 2,097,152 triangles 174 us with one thread per
+// cell, 190 with two; they cross near 262,144 (30.6 us both).
+uint32_t flux_threads(uint32_t bs, uint64_t cells) { return bs < 256 && cells <= (1u << 18) ? 2 * bs : bs; }
+int face_size(uint32_t bs) { return bs == 64 ? 0 : (bs == 128 ? 1 : 2); }
+}  // namespace
+
 hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t nblk = (g.N + bs - 1) / bs, per_xcd = (nblk + 7) / 8;
-    const dim3 grid(8 * per_xcd), block(bs);
+    const dim3 grid(8 * per_xcd), block(flux_threads(bs, g.N));
+    const size_t lds = (size_t)g.face_max[face_size(bs)] * 32;
     const bool pp = a.pp && a.op != kRhsOnly;
-#define MLR_FU(RSV)                                                                                           \
-    do {                                                                                                      \
-        if (pp) hipLaunchKernelGGL((flux_update_kernel<RSV, true>), grid, block, 0, stream, g, a, ph, per_xcd); \
-        else hipLaunchKernelGGL((flux_update_kernel<RSV, false>), grid, block, 0, stream, g, a, ph, per_xcd);   \
+    if (a.parts != 3 && a.op != kRhsOnly) return hipErrorInvalidValue;
+#define MLR_FU(RSV)                                                                                        \
+    do {                                                                                                   \
+        if (ph.viscous)                                                                                    \
+            hipLaunchKernelGGL((flux_update_kernel<RSV, false, true>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
+        else if (pp)                                                                                       \
+            hipLaunchKernelGGL((flux_update_kernel<RSV, true, false>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
+        else                                                                                               \
+            hipLaunchKernelGGL((flux_update_kernel<RSV, false, false>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
     } while (0)
     switch (a.riemann) {
     case 0: MLR_FU(0); break;
@@ -1506,29 +1518,6 @@ hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uin
     default: return hipErrorInvalidValue;
     }
 #undef MLR_FU
-    return hipGetLastError();
-}
-
-hipError_t rhs_parts(const Geom& g, const StageArgs& a, const Physics& ph, int parts, uint32_t bs,
-                     hipStream_t stream) {
-    if (parts == 3) return flux_update(g, a, ph, bs, stream);
-    if ((parts != 1 && parts != 2) || a.op != kRhsOnly) return hipErrorInvalidValue;
-    if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
-    const uint32_t nblk = (g.N + bs - 1) / bs, per_xcd = (nblk + 7) / 8;
-    const dim3 grid(8 * per_xcd), block(bs);
-#define MLR_PARTS(RSV)                                                                                        \
-    do {                                                                                                      \
-        if (parts == 1) hipLaunchKernelGGL((rhs_parts_kernel<RSV, 1>), grid, block, 0, stream, g, a, ph, per_xcd); \
-        else hipLaunchKernelGGL((rhs_parts_kernel<RSV, 2>), grid, block, 0, stream, g, a, ph, per_xcd);          \
-    } while (0)
-    switch (a.riemann) {
-    case 0: MLR_PARTS(0); break;
-    case 1: MLR_PARTS(1); break;
-    case 2: MLR_PARTS(2); break;
-    case 3: MLR_PARTS(3); break;
-    default: return hipErrorInvalidValue;
-    }
-#undef MLR_PARTS
     return hipGetLastError();
 }
 
@@ -1623,18 +1612,19 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
 }
 
 hipError_t flux_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const BatchStage& st, int riemann,
-                      const Physics& ph, uint32_t bs, hipStream_t stream) {
+                      const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
-    const dim3 grid(8 * per_xcd), block(bs);
-#define MLR_FB(RSV)                                                                                   \
-    do {                                                                                              \
-        if (st.pp)                                                                                    \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, true>), grid, block, 0, stream, cases, n_cases, st, \
-                               total_blocks, ph, per_xcd);                                            \
-        else                                                                                          \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, false>), grid, block, 0, stream, cases, n_cases, st, \
-                               total_blocks, ph, per_xcd);                                            \
+    const dim3 grid(8 * per_xcd), block(flux_threads(bs, (uint64_t)total_blocks * bs));
+    const size_t lds = (size_t)face_max * 32;
+#define MLR_FB(RSV)                                                                                     \
+    do {                                                                                                \
+        if (st.pp)                                                                                      \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, true>), grid, block, lds, stream, cases, n_cases, st, \
+                               total_blocks, ph, bs, per_xcd);                                          \
+        else                                                                                            \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, false>), grid, block, lds, stream, cases, n_cases, st, \
+                               total_blocks, ph, bs, per_xcd);                                          \
     } while (0)
     switch (riemann) {
     case 0: MLR_FB(0); break;
@@ -1667,9 +1657,12 @@ hipError_t finalize_batch(const CaseBufs* cases, int n_cases, double cfl, double
 namespace {
 template <int RS, bool TENO>
 hipError_t launch_step_persistent(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
-                                  const PersistentStep& ps, const Physics& ph, hipStream_t stream, int* grid_out) {
+                                  const PersistentStep& ps, uint32_t face_max, const Physics& ph, hipStream_t stream,
+                                  int* grid_out) {
     const void* fn = reinterpret_cast<const void*>(&ensemble_step_kernel<RS, TENO>);
-    const size_t lds = TENO ? 256 * 32 : 0;
+    // a block holds a TENO tile or a flux block's face fluxes
+    const size_t flux_lds = (size_t)face_max * 32;
+    const size_t lds = TENO && flux_lds < 256 * 32 ? 256 * 32 : flux_lds;
     int per_cu = 0, dev = 0, cus = 0;
     if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, lds); e != hipSuccess) return e;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
@@ -1689,12 +1682,14 @@ hipError_t launch_step_persistent(const CaseBufs* cases, int n_cases, uint32_t t
 }  // namespace
 
 hipError_t ensemble_step(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
-                         const PersistentStep& ps, int riemann, bool teno, const Physics& ph, hipStream_t stream,
-                         int* grid_out) {
+                         const PersistentStep& ps, int riemann, bool teno, uint32_t face_max, const Physics& ph,
+                         hipStream_t stream, int* grid_out) {
     if (n_cases < 1 || ps.n_stages < 1 || ps.n_stages > 4) return hipErrorInvalidValue;
 #define MLR_STEP(RSV)                                                                                          \
-    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_total, flux_total, ps, ph, stream, grid_out) \
-                : launch_step_persistent<RSV, false>(cases, n_cases, teno_total, flux_total, ps, ph, stream, grid_out)
+    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_total, flux_total, ps, face_max, ph, stream, \
+                                                    grid_out)                                                    \
+                : launch_step_persistent<RSV, false>(cases, n_cases, teno_total, flux_total, ps, face_max, ph, stream, \
+                                                     grid_out)
     switch (riemann) {
     case 0: MLR_STEP(0);
     case 1: MLR_STEP(1);

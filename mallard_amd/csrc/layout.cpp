@@ -441,9 +441,81 @@ void teno_matrices_of_cell(const Mesh& m, const TenoSpec& ts, uint32_t c,
 // ------------------------------------------------------------ layout
 uint64_t Layout::device_bytes() const {
     auto b = [](const auto& v) { return (uint64_t)v.size() * sizeof(v[0]); };
-    return b(volume) + b(nb) + b(info) + b(nx) + b(ny) + b(area) + b(dxn) + b(blk_off) + b(blk_ids) +
+    return b(volume) + b(nb) + b(info) + b(nx) + b(ny) + b(area) + b(dxn) + b(face_off) + b(face_c0) + b(face_c1) +
+           b(face_meta) + b(face_nx) + b(face_ny) + b(face_area) + b(cell_faces) + b(cell_sum) + b(blk_off) + b(blk_ids) +
            b(st_loc8) + b(st_loc16) + b(st_ta) +
            b(st_A) + b(fbasis);
+}
+
+// Face lists of the flux kernel (see Layout::face_off).
+void build_faces(Layout& L) {
+    const uint32_t N = L.N, S = L.S, B = Layout::kTileCells;
+    const uint32_t nblk = (N + B - 1) / B;
+    // slots that contribute to the residual, as a bit mask
+    auto active = [&](uint32_t c) {
+        const uint32_t code = (L.info[c] >> 8) & 0xFFu, nact = (L.info[c] >> 16) & 0x7u;
+        uint32_t m = 0;
+        for (uint32_t r = 0; r < nact; ++r) m |= 1u << ((code >> (2 * r)) & 3u);
+        return m;
+    };
+    // slot l of cell c lists its face unless the lower cell of the block does
+    auto lists = [&](uint32_t c, uint32_t l, uint32_t b) {
+        const size_t o = (size_t)l * N + c;
+        if (!((active(c) >> l) & 1u)) return false;
+        if (L.info[o] & kSlotBoundary) return true;
+        const uint32_t other = (uint32_t)L.nb[o];
+        return other / B != b || c < other;
+    };
+    L.face_off.assign(nblk + 1, 0);
+#pragma omp parallel for schedule(static)
+    for (int64_t b = 0; b < (int64_t)nblk; ++b) {
+        const uint32_t c0 = (uint32_t)b * B, c1 = std::min(N, c0 + B);
+        uint32_t n = 0;
+        for (uint32_t l = 0; l < S; ++l)
+            for (uint32_t c = c0; c < c1; ++c) n += lists(c, l, (uint32_t)b) ? 1u : 0u;
+        L.face_off[b + 1] = n;
+    }
+    for (uint32_t b = 0; b < nblk; ++b) L.face_off[b + 1] += L.face_off[b];
+    for (int k = 0; k < 3; ++k)
+        for (uint32_t b = 0; b < nblk; b += 1u << k)
+            L.face_max[k] = std::max(L.face_max[k], L.face_off[std::min(nblk, b + (1u << k))] - L.face_off[b]);
+    const size_t nf = L.face_off[nblk];
+    L.face_c0.resize(nf);
+    L.face_c1.resize(nf);
+    L.face_meta.resize(nf);
+    L.face_nx.resize(nf);
+    L.face_ny.resize(nf);
+    L.face_area.resize(nf);
+    L.cell_faces.assign(N, 0);
+    L.cell_sum.assign(N, 0);
+#pragma omp parallel for schedule(static)
+    for (int64_t b = 0; b < (int64_t)nblk; ++b) {
+        const uint32_t c0 = (uint32_t)b * B, c1 = std::min(N, c0 + B);
+        uint32_t n = 0;  // at most 64 S <= 256 entries: 8-bit positions
+        for (uint32_t l = 0; l < S; ++l)
+            for (uint32_t c = c0; c < c1; ++c) {
+                const size_t o = (size_t)l * N + c;
+                const uint32_t inf = L.info[o];
+                const bool bnd = (inf & kSlotBoundary) != 0;
+                const uint32_t side = (inf >> 2) & 1u;
+                if (l == 0) L.cell_sum[c] = ((inf >> 8) & 0xFFu) | (((inf >> 16) & 0x7u) << dev::kSumCountShift);
+                L.cell_sum[c] |= (side << (dev::kSumSideShift + l)) | ((bnd ? 1u : 0u) << (dev::kSumBoundaryShift + l));
+                if (!lists(c, l, (uint32_t)b)) continue;
+                const uint32_t other = (uint32_t)L.nb[o], nbs = inf & 3u;
+                const size_t e = (size_t)L.face_off[b] + n;
+                L.face_c0[e] = side ? other : c;
+                L.face_c1[e] = side ? c : other;
+                uint32_t meta = side ? nbs | (l << dev::kFaceSlot1Shift) : l | (nbs << dev::kFaceSlot1Shift);
+                if (bnd) meta |= dev::kFaceBoundary | (((inf >> 4) & 0xFu) << dev::kFaceBcShift);
+                L.face_meta[e] = (uint16_t)meta;
+                L.face_nx[e] = L.nx[o];
+                L.face_ny[e] = L.ny[o];
+                L.face_area[e] = L.area[o];
+                L.cell_faces[c] |= n << (8 * l);
+                if (!bnd && other / B == (uint32_t)b) L.cell_faces[other] |= n << (8 * nbs);
+                ++n;
+            }
+    }
 }
 
 // Per-block member lists and in-list positions (see Layout::blk_off).
@@ -620,6 +692,7 @@ Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::v
         L.info[j] |= (code << 8) | (nact << 16);
     }
     if (bad) fail("inconsistent cells_of_face / faces_of_cell connectivity");
+    build_faces(L);
 
     if (recon == Recon::FO) {
         L.Q = 1;

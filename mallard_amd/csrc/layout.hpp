@@ -65,6 +65,19 @@ struct Layout {
     std::vector<double> dcx, dcy;           // [S][N] centroid to neighbour centroid (face midpoint on boundaries)
     std::vector<double> mfx, mfy;           // [S][N] centroid to face midpoint
 
+    // Face lists of the flux kernel: block b = cells [64b, 64b+64). Entries
+    // face_off[b] .. face_off[b+1] hold every face of the block's cells that
+    // contributes to the residual, once: a face inside the block one entry, a
+    // face between two blocks one entry in each. Ordered by the slot and the
+    // cell that lists the face (the lower cell of a face inside the block).
+    std::vector<uint32_t> face_off;         // [n_blocks + 1]
+    std::vector<uint32_t> face_c0, face_c1; // side-0 and side-1 cell (side 0 again on boundaries)
+    std::vector<uint16_t> face_meta;        // dev::kFace* bits
+    std::vector<double> face_nx, face_ny, face_area;
+    std::vector<uint32_t> cell_faces;       // [N] in-block entry of each slot's face, 8 bits per slot
+    std::vector<uint32_t> cell_sum;         // [N] dev::kSum* bits: order, count and signs of the face sum
+    uint32_t face_max[3] = {0, 0, 0};       // most entries of 1, 2 and 4 consecutive blocks (from a multiple of it)
+
     // TENO (empty for FO): G = S + 1 stencils per cell, K = n_dof, M = cells per stencil.
     bool teno = false;
     int K = 0, M = 0, G = 0;

@@ -177,49 +177,56 @@ __device__ inline void riemann_flux(int type, int guard, double* F, double n0, d
     }
 }
 
-// Flux through one face point. Boundary states follow boundary_*.cpp; the
-// wall returns the pressure-only flux (boundary_wall_adiabatic.cpp:38-70).
-// On a boundary face Cl is the face state and Cr the state an extrapolation
-// boundary copies into its ghost (the face state itself in the reference).
+// The state beyond a boundary face: density rr and primitives Wr from the
+// face state Cl (primitives Wl) and the state Cr an extrapolation boundary
+// copies into its ghost (the face state itself in the reference). Boundary
+// states follow boundary_*.cpp. true: a wall, whose flux is the pressure
+// alone (wall_flux; boundary_wall_adiabatic.cpp:38-70), with Wl as the state.
+__device__ inline bool boundary_state(const Physics& ph, const BCParam& b, double n0, double n1, const double* Cl,
+                                      const double* Cr, const double* Wl, double& rr, double* Wr) {
+    rr = Cl[0];
+    if (b.type == 1) {  // extrapolation: the ghost is the state Cr
+        prims(ph, Cr, Wr);
+        rr = Cr[0];
+        return false;
+    }
+    for (int i = 0; i < 5; i++) Wr[i] = Wl[i];
+    if (b.type == 0) {  // symmetry: mirror the velocity (boundary_symmetry.cpp:38-69)
+        const double un = Wl[0] * n0 + Wl[1] * n1;
+        Wr[0] = Wl[0] - 2.0 * un * n0;
+        Wr[1] = Wl[1] - 2.0 * un * n1;
+    } else if (b.type == 2 || b.type == 5) {  // adiabatic wall (slip; no-slip adds viscous terms)
+        return true;
+    } else if (b.type == 3) {  // fixed u, p, T (boundary_upt.cpp:83-100)
+        rr = b.rho;
+        Wr[0] = b.u0; Wr[1] = b.u1; Wr[2] = b.p; Wr[3] = b.T; Wr[4] = b.h;
+    } else {  // p_out (boundary_p_out.cpp:57-100)
+        const double um = sqrt(Wl[0] * Wl[0] + Wl[1] * Wl[1]);
+        const double a = sqrt(ph.gamma * Wl[2] / Cl[0]);
+        const double pout = (um < a) ? b.p : Wl[2];
+        const double Tb = Wl[3];
+        const double rb = pout / (ph.R * Tb);
+        const double eb = ph.cv * Tb;
+        rr = rb;
+        Wr[2] = pout; Wr[4] = eb + pout / rb;
+    }
+    return false;
+}
+
+// Flux through one face point between the states Cl (side 0) and, on an
+// interior face, Cr (side 1); on a boundary face Cl is the face state and Cr
+// what an extrapolation boundary copies into its ghost.
 __device__ inline void point_flux(const Physics& ph, const BCParam* __restrict__ bct, int riemann, int guard,
                                   bool bnd, int bc, double n0,
                                   double n1, const double* Cl, const double* Cr, double* F) {
     double Wl[5], Wr[5];
-    double rr;
+    double rr = Cr[0];
+    bool wall = false;
     prims(ph, Cl, Wl);
-    if (!bnd) {
-        prims(ph, Cr, Wr);
-        rr = Cr[0];
-    } else {
-        const BCParam& b = bct[bc];
-        if (b.type == 0) {  // symmetry: mirror the velocity (boundary_symmetry.cpp:38-69)
-            for (int i = 0; i < 5; i++) Wr[i] = Wl[i];
-            const double un = Wl[0] * n0 + Wl[1] * n1;
-            Wr[0] = Wl[0] - 2.0 * un * n0;
-            Wr[1] = Wl[1] - 2.0 * un * n1;
-            rr = Cl[0];
-        } else if (b.type == 1) {  // extrapolation: the ghost is the state Cr
-            prims(ph, Cr, Wr);
-            rr = Cr[0];
-        } else if (b.type == 2 || b.type == 5) {  // adiabatic wall (slip; no-slip adds viscous terms)
-            F[0] = 0.0; F[1] = Wl[2] * n0; F[2] = Wl[2] * n1; F[3] = 0.0;
-            return;
-        } else if (b.type == 3) {  // fixed u, p, T (boundary_upt.cpp:83-100)
-            rr = b.rho;
-            Wr[0] = b.u0; Wr[1] = b.u1; Wr[2] = b.p; Wr[3] = b.T; Wr[4] = b.h;
-        } else {  // p_out (boundary_p_out.cpp:57-100)
-            const double um = sqrt(Wl[0] * Wl[0] + Wl[1] * Wl[1]);
-            const double a = sqrt(ph.gamma * Wl[2] / Cl[0]);
-            const double pout = (um < a) ? b.p : Wl[2];
-            const double Tb = Wl[3];
-            const double rb = pout / (ph.R * Tb);
-            const double eb = ph.cv * Tb;
-            const double hb = eb + pout / rb;
-            rr = rb;
-            Wr[0] = Wl[0]; Wr[1] = Wl[1]; Wr[2] = pout; Wr[3] = Tb; Wr[4] = hb;
-        }
-    }
+    if (!bnd) prims(ph, Cr, Wr);
+    else wall = boundary_state(ph, bct[bc], n0, n1, Cl, Cr, Wl, rr, Wr);
     riemann_flux(riemann, guard, F, n0, n1, Cl[0], Wl, Wl[2], ph.gamma, Wl[4], rr, Wr, Wr[2], ph.gamma, Wr[4]);
+    if (wall) { F[0] = 0.0; F[1] = Wl[2] * n0; F[2] = Wl[2] * n1; F[3] = 0.0; }
 }
 
 // ---------------------------------------------------------------- positivity

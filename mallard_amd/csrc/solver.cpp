@@ -305,6 +305,11 @@ void Solver::setup(Mesh&& mesh) {
     L_ = build_layout(mesh_, cfg_.recon, cfg_.teno, cfg_.bcs, cfg_.n_threads, /*allow_device=*/true);
     HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     upload();
+    // shapes of contexts that are not autotuned (programs that only call the
+    // residual): HLLC flux pass of 8,192 triangles 8.9 us with 128-cell
+    // blocks, 15.8 with 256; of 524,288 52 us with either; of 2,097,152 190
+    // against 174
+    if (!tuned_ && L_.N <= (1u << 18)) tune_.flux_block = 128;
     t_ = 0.0;
     step_ = 0;
     wall0_ = wall_seconds();
@@ -378,6 +383,15 @@ void Solver::upload() {
     up(ny_, L_.ny);
     up(area_, L_.area);
     up(dxn_, L_.dxn);
+    up(face_off_, L_.face_off);
+    up(face_c0_, L_.face_c0);
+    up(face_c1_, L_.face_c1);
+    up(face_meta_, L_.face_meta);
+    up(face_nx_, L_.face_nx);
+    up(face_ny_, L_.face_ny);
+    up(face_area_, L_.face_area);
+    up(cell_faces_, L_.cell_faces);
+    up(cell_sum_, L_.cell_sum);
     up(qw_, L_.qface_w);
     if (cfg_.viscous) {
         up(dcx_, L_.dcx);
@@ -486,6 +500,16 @@ dev::Geom Solver::geom() const {
     g.dcy = dcy_;
     g.mfx = mfx_;
     g.mfy = mfy_;
+    g.face_off = face_off_;
+    g.face_c0 = face_c0_;
+    g.face_c1 = face_c1_;
+    g.face_meta = face_meta_;
+    g.face_nx = face_nx_;
+    g.face_ny = face_ny_;
+    g.face_area = face_area_;
+    g.cell_faces = cell_faces_;
+    g.cell_sum = cell_sum_;
+    for (int k = 0; k < 3; ++k) g.face_max[k] = L_.face_max[k];
     return g;
 }
 
@@ -723,6 +747,7 @@ dev::StageArgs Solver::stage(int op, const double* Uin, double* Uout) const {
     a.fo = L_.teno ? 0 : 1;
     a.corrected = (L_.teno && L_.tspec.variant == TenoVariant::Corrected) ? 1 : 0;
     a.pp = cfg_.positivity ? 1 : 0;
+    a.parts = 3;
     a.Uin = Uin;
     a.Un = Un_;
     a.Uout = Uout;
@@ -1263,7 +1288,8 @@ void Solver::calc_rhs_device(const double* U_dev, int parts, double* rhs_dev) {
     if (cfg_.viscous) HIP_OK(dev::viscous_grad(geom(), U_dev, ph_, vp_, vg_, tune_.flux_block, stream_));
     dev::StageArgs a = stage(dev::kRhsOnly, U_dev, nullptr);
     a.rhs = rhs_dev;
-    HIP_OK(dev::rhs_parts(geom(), a, ph_, parts, tune_.flux_block, stream_));
+    a.parts = parts;
+    HIP_OK(dev::flux_update(geom(), a, ph_, tune_.flux_block, stream_));
     mark(kStatFluxMs);
 }
 

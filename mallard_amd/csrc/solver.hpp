@@ -227,6 +227,10 @@ private:
     double *dcx_ = nullptr, *dcy_ = nullptr, *mfx_ = nullptr, *mfy_ = nullptr, *vp_ = nullptr, *vg_ = nullptr;
     int32_t* nb_ = nullptr;
     uint32_t* info_ = nullptr;
+    // face lists of the flux kernel
+    uint32_t *face_off_ = nullptr, *face_c0_ = nullptr, *face_c1_ = nullptr, *cell_faces_ = nullptr, *cell_sum_ = nullptr;
+    uint16_t* face_meta_ = nullptr;
+    double *face_nx_ = nullptr, *face_ny_ = nullptr, *face_area_ = nullptr;
     dev::BCParam* bc_ = nullptr;
     uint8_t* loc8_ = nullptr;
     uint16_t* loc16_ = nullptr;
