@@ -378,13 +378,13 @@ class Solver:
         self._check(lib().mlr_set_state(self.h, _p(U), _p(prim)))
 
     def state(self):
-        U = np.zeros((self.n_cells, 4))
-        W = np.zeros((self.n_cells, 5))
+        U = np.empty((self.n_cells, 4))
+        W = np.empty((self.n_cells, 5))
         self._check(lib().mlr_get_state(self.h, _p(U), _p(W)))
         return U, W
 
     def calc_rhs(self):
-        r = np.zeros((self.n_cells, 4))
+        r = np.empty((self.n_cells, 4))
         self._check(lib().mlr_calc_rhs(self.h, _p(r)))
         return r
 
@@ -467,7 +467,7 @@ class Solver:
         """Residual of a caller's state over the interior faces (1), the
         boundary faces (2) or both (3), divided by the volume."""
         U = _f64(U)
-        r = np.zeros((self.n_cells, 4))
+        r = np.empty((self.n_cells, 4))
         self._check(lib().mlr_calc_rhs_of(self.h, _p(U), parts, _p(r)))
         return r
 
@@ -601,8 +601,8 @@ class Ensemble:
         self._check(lib().mlr_ensemble_init_quadrant(self.h, k, xs, ys, _p(_f64(states).reshape(16))))
 
     def state(self, k):
-        U = np.zeros((int(self.n_cells[k]), 4))
-        W = np.zeros((int(self.n_cells[k]), 5))
+        U = np.empty((int(self.n_cells[k]), 4))
+        W = np.empty((int(self.n_cells[k]), 5))
         self._check(lib().mlr_ensemble_get_state(self.h, k, _p(U), _p(W)))
         return U, W
 

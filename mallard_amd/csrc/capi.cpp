@@ -2,6 +2,7 @@
 // failures into status codes plus a per-context error string.
 #include "../../include/mallard_amd.h"
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -247,26 +248,21 @@ int mlr_get_sizes(const mlr_ctx* ctx, int64_t* s) {
 }
 
 static void quadrant_state(mlr::Solver& solver, double xs, double ys, const double* states) {
-    const mlr::Mesh& m = solver.mesh();
     const auto& ph_cfg = solver.config();
     const double R = ph_cfg.p_ref / (ph_cfg.T_ref * ph_cfg.rho_ref);
     const double cp = R * ph_cfg.gamma / (ph_cfg.gamma - 1.0);
     const double cv = cp / ph_cfg.gamma;
-    std::vector<double> U(4 * (size_t)m.n_cells), W(5 * (size_t)m.n_cells);
-    for (uint32_t c2 = 0; c2 < m.n_cells; ++c2) {
-        const bool r = m.cc(c2, 0) >= xs, t = m.cc(c2, 1) >= ys;
-        const int q = r ? (t ? 0 : 3) : (t ? 1 : 2);
+    mlr::dev::RegionRows rows{};
+    for (int q = 0; q < 4; ++q) {
         const double rho = states[4 * q], u0 = states[4 * q + 1], u1 = states[4 * q + 2], p = states[4 * q + 3];
         const double T = p / (rho * R);
         const double e = cv * T;
         const double E = e + 0.5 * (u0 * u0 + u1 * u1);
         const double h = e + p / rho;
-        double* Uc = &U[4 * (size_t)c2];
-        Uc[0] = rho; Uc[1] = rho * u0; Uc[2] = rho * u1; Uc[3] = rho * E;
-        double* Wc = &W[5 * (size_t)c2];
-        Wc[0] = u0; Wc[1] = u1; Wc[2] = p; Wc[3] = T; Wc[4] = h;
+        const double row[9] = {rho, rho * u0, rho * u1, rho * E, u0, u1, p, T, h};
+        std::copy(row, row + 9, rows.v[q]);
     }
-    solver.set_state(U.data(), W.data());
+    solver.set_regions(rows, [&](double x, double y) { return x >= xs ? (y >= ys ? 0 : 3) : (y >= ys ? 1 : 2); });
 }
 
 int mlr_init_quadrant(mlr_ctx* ctx, double xs, double ys, const double* states) {
@@ -277,7 +273,6 @@ int mlr_init_quadrant(mlr_ctx* ctx, double xs, double ys, const double* states) 
 int mlr_init_constant(mlr_ctx* ctx, const double* u, double p, double T) {
     if (!ctx || !u) return 1;
     return guarded(ctx, [&] {
-        const mlr::Mesh& m = ctx->solver.mesh();
         const auto& cf = ctx->solver.config();
         const double R = cf.p_ref / (cf.T_ref * cf.rho_ref);
         const double cp = R * cf.gamma / (cf.gamma - 1.0);
@@ -286,14 +281,10 @@ int mlr_init_constant(mlr_ctx* ctx, const double* u, double p, double T) {
         const double e = cv * T;
         const double E = e + 0.5 * (u[0] * u[0] + u[1] * u[1]);
         const double h = e + p / rho;
-        std::vector<double> U(4 * (size_t)m.n_cells), W(5 * (size_t)m.n_cells);
-        for (uint32_t c2 = 0; c2 < m.n_cells; ++c2) {
-            double* Uc = &U[4 * (size_t)c2];
-            Uc[0] = rho; Uc[1] = rho * u[0]; Uc[2] = rho * u[1]; Uc[3] = rho * E;
-            double* Wc = &W[5 * (size_t)c2];
-            Wc[0] = u[0]; Wc[1] = u[1]; Wc[2] = p; Wc[3] = T; Wc[4] = h;
-        }
-        ctx->solver.set_state(U.data(), W.data());
+        const double row[9] = {rho, rho * u[0], rho * u[1], rho * E, u[0], u[1], p, T, h};
+        mlr::dev::RegionRows rows{};
+        std::copy(row, row + 9, rows.v[0]);
+        ctx->solver.set_regions(rows, nullptr);
     });
 }
 

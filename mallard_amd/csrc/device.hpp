@@ -289,6 +289,24 @@ hipError_t riemann_points(int type, int guard, int64_t n, const double* nrm, con
 // vector updates of n doubles: kind 0 y = x (deep_copy), 1 y = y + a x
 // (axpy), 2 y = a x + b y (axpby)
 hipError_t vec_update(int kind, int64_t n, double a, const double* x, double b, double* y, hipStream_t stream);
+// State transfer between the reference's numbering (rows perm[j]) and the
+// solver's (rows j), on device arrays:
+// put_state: U[N][4] and, unless NULL, prim[N][5] (u, v, p, T, h) of the
+// reference's numbering into Un, prims and h; NULL primitives are computed
+// from U. take_state: the reverse; U or prim may be NULL.
+// put_regions: cell j takes row region[j] (row 0 where region is NULL) of
+// rows[][9] = (rho, rho u, rho v, rho E, u, v, p, T, h), n_rows <= 4.
+// rows4: dst[j] = src[perm[j]] (scatter 0) or dst[perm[j]] = src[j] (1) for rows of 4
+struct RegionRows {
+    double v[4][9];
+};
+hipError_t put_state(const Physics& ph, uint32_t N, const uint32_t* perm, const double* U, const double* prim,
+                     double* Un, double* prims, double* h, hipStream_t stream);
+hipError_t take_state(uint32_t N, const uint32_t* perm, const double* Un, const double* prims, const double* h,
+                      double* U, double* prim, hipStream_t stream);
+hipError_t put_regions(uint32_t N, const uint8_t* region, const RegionRows& rows, double* Un, double* prims,
+                       double* h, hipStream_t stream);
+hipError_t rows4(int scatter, uint32_t N, const uint32_t* perm, const double* src, double* dst, hipStream_t stream);
 // The Riemann operator on HOST arrays (same layouts): stages the points
 // through device memory allocated for the call, on the null stream; throws
 // mlr::Error on failure

@@ -40,16 +40,6 @@ T lookup_enum(const std::string& key, std::initializer_list<std::pair<const char
     fail("Unknown " + what + ": " + key + ".");
 }
 
-// physics.h:852-867 on the host (same operation order as the device)
-void host_prims(const dev::Physics& ph, const double* U, double* W) {
-    const double rho = U[0];
-    const double u0 = U[1] / rho, u1 = U[2] / rho;
-    const double E = U[3] / rho;
-    const double e = E - 0.5 * (u0 * u0 + u1 * u1);
-    const double p = std::fmax(ph.p_min, std::fmin(ph.p_max, (ph.gamma - 1.0) * rho * e));
-    W[0] = u0; W[1] = u1; W[2] = p; W[3] = e / ph.cv; W[4] = e + p / rho;
-}
-
 constexpr int64_t kDtHistCap = 1 << 20;
 
 }  // namespace
@@ -379,6 +369,7 @@ void Solver::upload() {
     up(volume_, L_.volume);
     up(nb_, L_.nb);
     up(info_, L_.info);
+    up(perm_, L_.perm);
     up(nx_, L_.nx);
     up(ny_, L_.ny);
     up(area_, L_.area);
@@ -459,13 +450,15 @@ void Solver::upload() {
         return p;
     };
     Un_ = dz(4 * N);
-    Ua_ = dz(4 * N);
+    // the stage buffers in one piece: between steps they hold nothing a step
+    // reads before it writes it, and carry states to and from the host
+    Ua_ = dz(12 * N);
+    Ub_ = Ua_ + 4 * N;
+    W_ = Ua_ + 8 * N;
     if (cfg_.viscous) {
         vp_ = dz(4 * N);
         vg_ = dz(6 * N);
     }
-    Ub_ = dz(4 * N);
-    W_ = dz(4 * N);
     prims_ = dz(4 * N);
     h_ = dz(N);
     rhs_ = dz(4 * N);
@@ -480,6 +473,8 @@ void Solver::upload() {
     gated_ = (uint32_t*)dz((gated_slots_ + 1) / 2);
     dec_ = (uint8_t*)dalloc(N);
     HIP_OK(hipMemset(dec_, 0, N));
+    // the fills run on the null stream, which stream_ does not wait for
+    HIP_OK(hipStreamSynchronize(nullptr));
 }
 
 dev::Geom Solver::geom() const {
@@ -1173,72 +1168,69 @@ void Solver::take_step() {
 void Solver::calc_rhs(double* rhs_ref) {
     if (L_.teno) launch_teno(Un_);
     launch_flux(dev::kRhsOnly, Un_, nullptr);
-    std::vector<double> r(4 * (size_t)L_.N);
-    HIP_OK(hipMemcpyAsync(r.data(), rhs_, r.size() * 8, hipMemcpyDeviceToHost, stream_));
-    synchronize();
-    for (uint32_t j = 0; j < L_.N; ++j) std::memcpy(&rhs_ref[4 * (size_t)L_.perm[j]], &r[4 * (size_t)j], 32);
+    download_rows(rhs_, rhs_ref);
 }
 
+// The host-facing copies below stage rows of the reference's numbering in the
+// stage buffers (9 doubles per cell of their 12) and renumber them on the GPU.
 void Solver::set_state(const double* U, const double* prim5) {
     const size_t N = L_.N;
-    std::vector<double> u(4 * N), w(4 * N), h(N);
-    for (uint32_t j = 0; j < N; ++j) {
-        const uint32_t c = L_.perm[j];
-        std::memcpy(&u[4 * (size_t)j], &U[4 * (size_t)c], 32);
-        double W5[5];
-        if (prim5) std::memcpy(W5, &prim5[5 * (size_t)c], 40);
-        else host_prims(ph_, &U[4 * (size_t)c], W5);
-        std::memcpy(&w[4 * (size_t)j], W5, 32);
-        h[j] = W5[4];
-    }
-    HIP_OK(hipMemcpy(Un_, u.data(), u.size() * 8, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(prims_, w.data(), w.size() * 8, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(h_, h.data(), h.size() * 8, hipMemcpyHostToDevice));
+    double *u = Ua_, *w = Ua_ + 4 * N;
+    synchronize();
+    HIP_OK(hipMemcpy(u, U, 4 * N * 8, hipMemcpyHostToDevice));
+    if (prim5) HIP_OK(hipMemcpy(w, prim5, 5 * N * 8, hipMemcpyHostToDevice));
+    HIP_OK(dev::put_state(ph_, L_.N, perm_, u, prim5 ? w : nullptr, Un_, prims_, h_, stream_));
+    synchronize();
 }
 
 void Solver::get_state(double* U, double* prim5) {
     const size_t N = L_.N;
-    std::vector<double> u(4 * N), w(4 * N), h(N);
+    double *u = Ua_, *w = Ua_ + 4 * N;
+    HIP_OK(dev::take_state(L_.N, perm_, Un_, prims_, h_, U ? u : nullptr, prim5 ? w : nullptr, stream_));
     synchronize();
-    HIP_OK(hipMemcpy(u.data(), Un_, u.size() * 8, hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(w.data(), prims_, w.size() * 8, hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(h.data(), h_, h.size() * 8, hipMemcpyDeviceToHost));
-    for (uint32_t j = 0; j < N; ++j) {
-        const uint32_t c = L_.perm[j];
-        if (U) std::memcpy(&U[4 * (size_t)c], &u[4 * (size_t)j], 32);
-        if (prim5) {
-            std::memcpy(&prim5[5 * (size_t)c], &w[4 * (size_t)j], 32);
-            prim5[5 * (size_t)c + 4] = h[j];
-        }
+    if (U) HIP_OK(hipMemcpy(U, u, 4 * N * 8, hipMemcpyDeviceToHost));
+    if (prim5) HIP_OK(hipMemcpy(prim5, w, 5 * N * 8, hipMemcpyDeviceToHost));
+}
+
+void Solver::set_regions(const dev::RegionRows& rows, const std::function<int(double, double)>& region_of) {
+    const uint32_t N = L_.N;
+    std::vector<uint8_t> region;
+    if (region_of) {
+        region.resize(N);
+#pragma omp parallel for schedule(static) if (N > 65536)
+        for (int64_t j = 0; j < (int64_t)N; ++j)
+            region[(size_t)j] = (uint8_t)region_of(L_.centroid[2 * (size_t)j], L_.centroid[2 * (size_t)j + 1]);
+        HIP_OK(hipMemcpyAsync(Ua_, region.data(), N, hipMemcpyHostToDevice, stream_));
     }
+    HIP_OK(dev::put_regions(N, region_of ? reinterpret_cast<const uint8_t*>(Ua_) : nullptr, rows, Un_, prims_, h_,
+                            stream_));
+    synchronize();
 }
 
 // solver_initialize.cpp:35-186
 void Solver::init_solution() {
-    const uint32_t N = mesh_.n_cells;
-    std::vector<double> U(4 * (size_t)N), W(5 * (size_t)N);
-    auto put = [&](uint32_t c, double rho, double u0, double u1, double p, double T) {
+    // conserved state and primitives of one point, row[9]
+    auto state_row = [&](double* row, double rho, double u0, double u1, double p, double T) {
         const double e = ph_.cv * T;
         const double E = e + 0.5 * (u0 * u0 + u1 * u1);
         const double h = e + p / rho;
-        double* Uc = &U[4 * (size_t)c];
-        Uc[0] = rho; Uc[1] = rho * u0; Uc[2] = rho * u1; Uc[3] = rho * E;
-        double* Wc = &W[5 * (size_t)c];
-        Wc[0] = u0; Wc[1] = u1; Wc[2] = p; Wc[3] = T; Wc[4] = h;
+        row[0] = rho; row[1] = rho * u0; row[2] = rho * u1; row[3] = rho * E;
+        row[4] = u0; row[5] = u1; row[6] = p; row[7] = T; row[8] = h;
     };
     const InitSpec& I = cfg_.init;
+    dev::RegionRows rows{};
     if (I.kind == InitSpec::Constant) {
-        const double rho = I.p / (ph_.R * I.T);
-        for (uint32_t c = 0; c < N; ++c) put(c, rho, I.u[0], I.u[1], I.p, I.T);
+        state_row(rows.v[0], I.p / (ph_.R * I.T), I.u[0], I.u[1], I.p, I.T);
+        set_regions(rows, nullptr);
     } else if (I.kind == InitSpec::Quadrant) {
-        for (uint32_t c = 0; c < N; ++c) {
-            const bool r = mesh_.cc(c, 0) >= I.xs, t = mesh_.cc(c, 1) >= I.ys;
-            const int q = r ? (t ? 0 : 3) : (t ? 1 : 2);
+        for (int q = 0; q < 4; ++q) {
             const double* s = &I.states[4 * q];
-            const double rho = s[0], p = s[3];
-            put(c, rho, s[1], s[2], p, p / (rho * ph_.R));
+            state_row(rows.v[q], s[0], s[1], s[2], s[3], s[3] / (s[0] * ph_.R));
         }
+        set_regions(rows, [&](double x, double y) { return x >= I.xs ? (y >= I.ys ? 0 : 3) : (y >= I.ys ? 1 : 2); });
     } else {
+        const uint32_t N = mesh_.n_cells;
+        std::vector<double> U(4 * (size_t)N), W(5 * (size_t)N);
         Expression ux(I.u_expr[0]), uy(I.u_expr[1]);
         std::unique_ptr<Expression> er, ep, eT;
         if (!I.rho_expr.empty()) er.reset(new Expression(I.rho_expr));
@@ -1255,21 +1247,28 @@ void Solver::init_solution() {
             else if (er && eT) p = rho * ph_.R * T;
             else if (ep && eT) rho = p / (ph_.R * T);
             else fail("Exactly two of rho, p, and T must be specified for initialization: analytical.");
-            put(c, rho, u0, u1, p, T);
+            double row[9];
+            state_row(row, rho, u0, u1, p, T);
+            std::memcpy(&U[4 * (size_t)c], row, 32);
+            std::memcpy(&W[5 * (size_t)c], row + 4, 40);
         }
+        set_state(U.data(), W.data());
     }
-    set_state(U.data(), W.data());
 }
 
 void Solver::get_face_values(double* out) { face_values_from(Un_, out); }
 
 void Solver::upload_state(const double* U_ref, double* dst_dev) {
     if (!U_ref) fail("state is NULL");
-    const size_t N = L_.N;
-    std::vector<double> u(4 * N);
-    for (uint32_t j = 0; j < N; ++j) std::memcpy(&u[4 * (size_t)j], &U_ref[4 * (size_t)L_.perm[j]], 32);
     synchronize();
-    HIP_OK(hipMemcpy(dst_dev, u.data(), u.size() * 8, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(Ub_, U_ref, 32 * (size_t)L_.N, hipMemcpyHostToDevice));
+    HIP_OK(dev::rows4(0, L_.N, perm_, Ub_, dst_dev, stream_));
+}
+
+void Solver::download_rows(const double* src_dev, double* out_ref) {
+    HIP_OK(dev::rows4(1, L_.N, perm_, src_dev, Ub_, stream_));
+    synchronize();
+    HIP_OK(hipMemcpy(out_ref, Ub_, 32 * (size_t)L_.N, hipMemcpyDeviceToHost));
 }
 
 // The stage buffer Ua_ carries the caller's state: between steps it holds
@@ -1297,10 +1296,7 @@ void Solver::calc_rhs_of(const double* U_ref, int parts, double* rhs_ref) {
     if (!rhs_ref) fail("rhs is NULL");
     upload_state(U_ref, Ua_);
     calc_rhs_device(Ua_, parts, rhs_);
-    std::vector<double> r(4 * (size_t)L_.N);
-    HIP_OK(hipMemcpyAsync(r.data(), rhs_, r.size() * 8, hipMemcpyDeviceToHost, stream_));
-    synchronize();
-    for (uint32_t j = 0; j < L_.N; ++j) std::memcpy(&rhs_ref[4 * (size_t)L_.perm[j]], &r[4 * (size_t)j], 32);
+    download_rows(rhs_, rhs_ref);
 }
 
 void Solver::face_values_from(const double* cells_dev, double* out) {

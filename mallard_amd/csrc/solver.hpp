@@ -5,6 +5,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -104,6 +105,10 @@ public:
     // reference-numbered host state I/O
     void set_state(const double* U, const double* prim5);
     void get_state(double* U, double* prim5);
+    // a state of up to 4 uniform regions: row r of rows (rho, rho u, rho v,
+    // rho E, u, v, p, T, h) for the cells of region r; region_of(x, y) at the
+    // cells' centroids (NULL: every cell takes row 0)
+    void set_regions(const dev::RegionRows& rows, const std::function<int(double, double)>& region_of);
     void init_solution();
     void calc_rhs(double* rhs_ref);                 // R(Un) into host rhs (reference order)
     double calc_dt();                               // solver.cpp:580-590
@@ -211,6 +216,7 @@ private:
     void finish_steps(int64_t s0, int64_t n, double* dts_out);
     void face_values_from(const double* cells_dev, double* out);  // fs_ (TENO) or the cell states (FO)
     void upload_state(const double* U_ref, double* dst_dev);     // reference numbering -> dst_dev
+    void download_rows(const double* src_dev, double* out_ref);  // rows of 4 -> reference numbering
 
     Config cfg_;
     Mesh mesh_;
@@ -227,6 +233,7 @@ private:
     double *dcx_ = nullptr, *dcy_ = nullptr, *mfx_ = nullptr, *mfy_ = nullptr, *vp_ = nullptr, *vg_ = nullptr;
     int32_t* nb_ = nullptr;
     uint32_t* info_ = nullptr;
+    uint32_t* perm_ = nullptr;  // reference row of each cell
     // face lists of the flux kernel
     uint32_t *face_off_ = nullptr, *face_c0_ = nullptr, *face_c1_ = nullptr, *cell_faces_ = nullptr, *cell_sum_ = nullptr;
     uint16_t* face_meta_ = nullptr;
