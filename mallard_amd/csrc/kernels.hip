@@ -56,6 +56,29 @@ __device__ inline double pressure_raw(double gamma, const double* u) {
     return (gamma - 1.0) * (u[3] - 0.5 * (u[1] * u[1] + u[2] * u[2]) / u[0]);
 }
 
+// The largest step tt in [0, 1] from the cell mean Uc toward the face state u
+// that keeps density and pressure at or above eps (Zhang & Shu 2010, the
+// pressure by bisection), in the oracle's order.
+__device__ inline double point_limit(double gamma, const double* Uc, const double* u, double eps) {
+    double wv[4];
+    double tt = 1.0;
+    if (u[0] < eps) tt = (Uc[0] - eps) / (Uc[0] - u[0]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) wv[k] = Uc[k] + tt * (u[k] - Uc[k]);
+    if (pressure_raw(gamma, wv) < eps) {
+        double lo = 0.0, hi = tt;
+        for (int it = 0; it < 40; it++) {
+            const double mid = 0.5 * (lo + hi);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) wv[k] = Uc[k] + mid * (u[k] - Uc[k]);
+            if (pressure_raw(gamma, wv) < eps) hi = mid;
+            else lo = mid;
+        }
+        tt = lo;
+    }
+    return tt;
+}
+
 // ------------------------------------------------------------ quad exchange
 // The 4 lanes of a quad serve one cell. DPP quad permutations move values
 // between them in registers (no LDS, so occupancy is set by VGPRs alone).
@@ -82,17 +105,6 @@ __device__ inline void quad_transpose(const double* x, double* out, int q) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) out[j] = sel4(r, (q - j) & 3);
 }
-// out[j] = f of quad lane j.
-__device__ inline void quad_gather(double f, double* out, int q) {
-    double r[4];
-    r[0] = f;
-    r[1] = qperm<kRot1>(f);
-    r[2] = qperm<kRot2>(f);
-    r[3] = qperm<kRot3>(f);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = sel4(r, (q - j) & 3);
-}
-
 // ------------------------------------------------------------ derived tables
 // The target cell's frame: node 0 and the inverse of the Jacobian of its
 // map from the reference triangle, as the precompute forms them.
@@ -290,23 +302,6 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
             wave_sync();
         } else {
             quad_transpose(x, out, q);
-        }
-    };
-    // out[j] = f[fq] of quad lane j, fq < FQ
-    auto gather = [&](const double* f, double (*out)[4]) {
-        if constexpr (kLdsX && FQ <= 4) {
-            const uint32_t tid = threadIdx.x, base = tid & ~3u;
-#pragma unroll
-            for (int fq = 0; fq < FQ; ++fq) xbuf[fq * kXs + tid] = f[fq];
-            wave_sync();
-#pragma unroll
-            for (int fq = 0; fq < FQ; ++fq)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) out[fq][j] = xbuf[fq * kXs + base + j];
-            wave_sync();
-        } else {
-#pragma unroll
-            for (int fq = 0; fq < FQ; ++fq) quad_gather(f[fq], out[fq], q);
         }
     };
     // the member update a += A+_i (ta_i (u_i - u_c)) of member i of this
@@ -536,35 +531,23 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     const int v = q;
 
     if (t.variant != 0) {
-        // positivity scaling of the cell's face states (Zhang & Shu 2010),
-        // computed redundantly by the 4 lanes, in the oracle's order
-        double uf[FQ][4];
-        gather(f, uf);
-        const double Uc[4] = {uc.v[0], uc.v[1], uc.v[2], uc.v[3]};
-        const double pc = pressure_raw(ph.gamma, Uc);
-        const double eps = fmin(1.0e-13, fmin(Uc[0], pc));
-        double theta = 1.0;
+        // positivity scaling of the cell's face states (Zhang & Shu 2010):
+        // quad lane q takes the limits of face points q and q + 4 (the
+        // 40-step bisection is a serial chain, and the quad's four chains
+        // run side by side), the smallest holds for the cell
+        const double pc = pressure_raw(ph.gamma, uc.v);
+        const double eps = fmin(1.0e-13, fmin(uc.v[0], pc));
+        double limit = 1.0;
 #pragma unroll
-        for (int fq = 0; fq < FQ; ++fq) {
-            const double* u = uf[fq];
-            double wv[4];
-            double tt = 1.0;
-            if (u[0] < eps) tt = (Uc[0] - eps) / (Uc[0] - u[0]);
+        for (int h = 0; h < FQ; h += 4) {
+            double x[4], u[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) wv[k] = Uc[k] + tt * (u[k] - Uc[k]);
-            if (pressure_raw(ph.gamma, wv) < eps) {
-                double lo = 0.0, hi = tt;
-                for (int it = 0; it < 40; it++) {
-                    const double mid = 0.5 * (lo + hi);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) wv[k] = Uc[k] + mid * (u[k] - Uc[k]);
-                    if (pressure_raw(ph.gamma, wv) < eps) hi = mid;
-                    else lo = mid;
-                }
-                tt = lo;
-            }
-            theta = fmin(theta, tt);
+            for (int j = 0; j < 4; ++j) x[j] = h + j < FQ ? f[h + j < FQ ? h + j : 0] : 0.0;
+            exchange(x, u);
+            if (h + q < FQ) limit = fmin(limit, point_limit(ph.gamma, uc.v, u, eps));
         }
+        const double other = fmin(qperm<kRot1>(limit), fmin(qperm<kRot2>(limit), qperm<kRot3>(limit)));
+        const double theta = fmin(limit, other);
         if (theta < 1.0)
 #pragma unroll
             for (int fq = 0; fq < FQ; ++fq) f[fq] = ucv + theta * (f[fq] - ucv);
