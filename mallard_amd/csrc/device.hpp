@@ -354,13 +354,22 @@ hipError_t ind_features(const Geom& g, const Teno& t, const double* U, const uin
                         uint16_t* X, float* y, uint64_t base, hipStream_t stream);
 hipError_t ind_infer(const ind::Net& net, const uint16_t* X, uint64_t n, float* z, hipStream_t stream);
 int ind_train_blocks(uint32_t B);
-// gradient of the weighted mean BCE over rows idx[0..B) (part: ind_train_blocks(B) x kNParams)
-hipError_t ind_grad(const ind::Net& net, const float* W2f, const uint16_t* X, const float* y, const uint32_t* idx,
+// The rows of a training batch: idx[i] where idx is given, else entries of
+// pool[n_pool] drawn by a hash of (seed, step, i).
+struct TrainBatch {
+    const uint32_t* idx;
+    const uint32_t* pool;
+    uint64_t n_pool, seed, step;
+};
+// gradient of the weighted mean BCE over a batch of B rows (part: ind_train_blocks(B) x kNParams)
+hipError_t ind_grad(const ind::Net& net, const float* W2f, const uint16_t* X, const float* y, const TrainBatch& batch,
                     uint32_t B, float pos_w, float neg_w, float* part, float* loss_part, float* grad, float* loss,
                     hipStream_t stream);
-hipError_t ind_adam(float* theta, float* m, float* v, const float* grad, float lr, int step, hipStream_t stream);
-hipError_t ind_batch(const uint32_t* pool, uint64_t n_pool, uint64_t seed, uint64_t step, uint32_t B,
-                     uint32_t* idx, hipStream_t stream);
+// one training step: the gradient, Adam on theta and the updated network
+// packed into net_buf (packed by net_pack before the first step)
+hipError_t ind_train_step(void* net_buf, const uint16_t* X, const float* y, const TrainBatch& batch, uint32_t B,
+                          float pos_w, float neg_w, float* part, float* loss_part, float* loss, float* theta, float* m,
+                          float* v, float lr, int step, hipStream_t stream);
 // Streaming bandwidth probes: kind 0 copies `bytes` from src to dst, kind 1
 // reads them (dst receives stream_probe_threads(bytes) doubles).
 uint32_t stream_probe_threads(size_t bytes);

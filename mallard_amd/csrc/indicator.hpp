@@ -165,15 +165,6 @@ __device__ inline double scale_feature(double s) { return s > 0.0 ? fmax(-2.0, (
 __device__ inline double inv_scale(double s) { return s > 0.0 ? 1.0 / s : 0.0; }
 __device__ inline double pattern_feature(double d, double is) { return d * is; }
 
-__device__ inline v4s pack4(const uint16_t* f) {
-    v4s x;
-    x[0] = (short)f[0];
-    x[1] = (short)f[1];
-    x[2] = (short)f[2];
-    x[3] = (short)f[3];
-    return x;
-}
-
 // Block-wide copy of the network's inference part into LDS (the caller
 // synchronises before use) and the view of that copy.
 __device__ inline void stage_net(const Net& net, unsigned char* lds) {

@@ -96,8 +96,9 @@ void mlp_grad(const float* params, const Dataset& ds, const uint32_t* idx, uint3
     hip_ok(hipMemcpy(didx.p, idx, B * sizeof(uint32_t), hipMemcpyHostToDevice), "hipMemcpy");
     DeviceNet net;
     net.pack(theta.as<float>(), st.s);
-    hip_ok(dev::ind_grad(net.net, net.W2f, ds.X, ds.y, didx.as<uint32_t>(), B, pos_w, neg_w, part.as<float>(),
-                         lpart.as<float>(), dgrad.as<float>(), dloss.as<float>(), st.s), "ind_grad");
+    hip_ok(dev::ind_grad(net.net, net.W2f, ds.X, ds.y, dev::TrainBatch{didx.as<uint32_t>(), nullptr, 0, 0, 0}, B, pos_w,
+                         neg_w, part.as<float>(), lpart.as<float>(), dgrad.as<float>(), dloss.as<float>(), st.s),
+           "ind_grad");
     hip_ok(hipStreamSynchronize(st.s), "sync");
     hip_ok(hipMemcpy(grad, dgrad.p, kIndParams * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
     hip_ok(hipMemcpy(loss, dloss.p, sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
@@ -111,24 +112,21 @@ void mlp_train(float* params, const Dataset& ds, const uint32_t* pool, uint64_t 
     Stream st;
     const int nblk = dev::ind_train_blocks(B);
     DBuf theta(kIndParams * sizeof(float)), m(kIndParams * sizeof(float)), v(kIndParams * sizeof(float));
-    DBuf dpool(n_pool * sizeof(uint32_t)), didx(B * sizeof(uint32_t));
+    DBuf dpool(n_pool * sizeof(uint32_t));
     DBuf part((size_t)nblk * kIndParams * sizeof(float)), lpart(nblk * sizeof(float));
-    DBuf dgrad(kIndParams * sizeof(float)), dloss((size_t)steps * sizeof(float));
+    DBuf dloss((size_t)steps * sizeof(float));
     hip_ok(hipMemcpy(theta.p, params, kIndParams * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
     hip_ok(hipMemcpy(dpool.p, pool, n_pool * sizeof(uint32_t), hipMemcpyHostToDevice), "hipMemcpy");
     hip_ok(hipMemsetAsync(m.p, 0, kIndParams * sizeof(float), st.s), "memset");
     hip_ok(hipMemsetAsync(v.p, 0, kIndParams * sizeof(float), st.s), "memset");
     DeviceNet net;
-    for (int k = 0; k < steps; ++k) {
-        net.pack(theta.as<float>(), st.s);
-        hip_ok(dev::ind_batch(dpool.as<uint32_t>(), n_pool, seed, (uint64_t)k, B, didx.as<uint32_t>(), st.s),
-               "ind_batch");
-        hip_ok(dev::ind_grad(net.net, net.W2f, ds.X, ds.y, didx.as<uint32_t>(), B, pos_w, neg_w,
-                             part.as<float>(), lpart.as<float>(), dgrad.as<float>(), dloss.as<float>() + k, st.s),
-               "ind_grad");
-        hip_ok(dev::ind_adam(theta.as<float>(), m.as<float>(), v.as<float>(), dgrad.as<float>(), lr, k + 1, st.s),
-               "ind_adam");
-    }
+    net.pack(theta.as<float>(), st.s);
+    for (int k = 0; k < steps; ++k)
+        hip_ok(dev::ind_train_step(net.buf.p, ds.X, ds.y,
+                                   dev::TrainBatch{nullptr, dpool.as<uint32_t>(), n_pool, seed, (uint64_t)k}, B, pos_w,
+                                   neg_w, part.as<float>(), lpart.as<float>(), dloss.as<float>() + k,
+                                   theta.as<float>(), m.as<float>(), v.as<float>(), lr, k + 1, st.s),
+               "ind_train_step");
     hip_ok(hipStreamSynchronize(st.s), "sync");
     hip_ok(hipMemcpy(params, theta.p, kIndParams * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
     if (loss_hist)
