@@ -105,9 +105,11 @@ struct Teno {
     const uint16_t* loc16;     // [G][M-1][N] otherwise (<= 1024 cells)
     const uint32_t* blk_off;   // [n_blocks + 1]
     const int32_t* blk_ids;    // tile lists, ascending cell ids
+    uint32_t tile_max;         // longest tile list
     const double* ta;
     const double* A;
     const double* fbasis;
+    const double* oi;   // OI in device memory (streamed passes)
     double OI[81];      // (K-1) x (K-1) block of the oscillation indicator, row-major
     // learned indicator gate: when gate != 0 a cell the network judges smooth
     // takes the central stencil alone; gated counts smooth cells, one
@@ -205,8 +207,8 @@ struct BatchStage {
 // Launch shapes an autotuner picks per mesh. Every choice gives identical
 // results; only the speed differs.
 struct Tune {
-    int32_t teno_occ = 0;       // TENO waves per SIMD targeted with stencil factor 2: 0 (the
-                                // compiler's choice); 5 or 6 at p = 2, 4 or 5 for plain p = 3
+    int32_t teno_occ = 0;       // TENO waves per SIMD targeted at p = 2 with stencil factor 2:
+                                // 0 (the compiler's choice), 5 or 6 (4 too with the derived basis)
     uint32_t flux_block = 256;  // cells per flux / stage-update block: 64, 128 or 256
     uint32_t spec_block = 256;  // cells per spectral-radius block: 64, 128 or 256
     int32_t teno_occ_reuse = 0; // the same target for gated passes that reuse recorded decisions

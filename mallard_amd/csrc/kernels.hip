@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "ddpow.hpp"
 #include "device.hpp"
@@ -146,6 +147,80 @@ __device__ inline double legendre_le2(int p, double x) {
     return p == 0 ? 1.0 : (p == 1 ? x : p2);
 }
 
+// ------------------------------------------------------------ streamed tables
+template <int I, int N, typename F>
+__device__ __forceinline__ void each_index_from(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        each_index_from<I + 1, N>(f);
+    }
+}
+template <int N, typename F>
+__device__ __forceinline__ void each_index(F&& f) {
+    each_index_from<0, N>(f);
+}
+
+// A wave's member tables through LDS. For each member the wave's 64 lanes (16
+// cells x 4 stencils) need KP rows of A+, one of areas and one of positions,
+// each 64 consecutive entries. Loads that write LDS directly (16 bytes a
+// lane, two rows an instruction) fetch SD members ahead without holding
+// registers, so the loads in flight do not compete with the accumulators.
+// A wave reads only its own slots: it waits for its own loads (they complete
+// in order), and for its reads of a slot before that slot is loaded again.
+template <int KP, int MP, typename IdxT, int SD>
+struct MemberStream {
+    static constexpr int kRows = KP + 1;                            // A+ rows and the areas
+    static constexpr int kSlot = kRows * 512 + 64 * (int)sizeof(IdxT);
+    static constexpr int kLoads = kRows / 2 + 1;                    // instructions per member
+    // the next member to load: the wave's A+ rows and positions, and this
+    // lane's part of the last two rows (an A+ row for the lower half of the
+    // lanes, the areas for the upper)
+    const unsigned char *rows, *pos, *last;
+    uint32_t lane_rows, lane_pos, last_step;
+    unsigned char *base, *next;
+
+    __device__ __forceinline__ void init(const Teno& t, uint32_t lb, unsigned char* slots) {
+        static_assert(SD == 0 || kRows % 2 == 0, "row pairs");
+        const uint32_t lane = threadIdx.x & 63u, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        base = slots + (size_t)w * SD * kSlot;
+        next = base;
+        const bool upper = lane >= 32;
+        rows = reinterpret_cast<const unsigned char*>(t.A + teno_a_off(lb, MP, KP, 0, 0, 16 * w, 0));
+        lane_rows = (lane >> 5) * 2048 + (lane & 31) * 16;
+        last = upper ? reinterpret_cast<const unsigned char*>(t.ta + teno_mem_off(lb, MP, 0, 16 * w, 0)) +
+                           (lane & 31) * 16
+                     : rows + (kRows / 2 - 1) * 4096 + lane * 16;
+        last_step = upper ? 2048 : KP * 2048;
+        const unsigned char* loc = sizeof(IdxT) == 1 ? t.loc8 : reinterpret_cast<const unsigned char*>(t.loc16);
+        pos = loc + teno_mem_off(lb, MP, 0, 16 * w, 0) * sizeof(IdxT);
+        lane_pos = lane * 16;
+    }
+    __device__ __forceinline__ unsigned char* slot(int i) const { return base + (i % SD) * kSlot; }
+    static __device__ __forceinline__ void load16(const unsigned char* src, unsigned char* dst) {
+        __builtin_amdgcn_global_load_lds(const_cast<unsigned char*>(src),
+                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+    __device__ __forceinline__ void issue() {
+#pragma unroll
+        for (int n = 0; n < kRows / 2 - 1; ++n) load16(rows + n * 4096 + lane_rows, next + n * 1024);
+        load16(last, next + (kRows / 2 - 1) * 1024);
+        if (lane_pos < 64 * sizeof(IdxT)) load16(pos + lane_pos, next + kRows * 512);
+        rows += KP * 2048;
+        last += last_step;
+        pos += 256 * sizeof(IdxT);
+        next = next == base + (SD - 1) * kSlot ? base : next + kSlot;
+    }
+    // member I's loads are complete: all but those of the members issued after it
+    template <int I>
+    __device__ __forceinline__ void wait() const {
+        constexpr int kAfter = MP - 1 - I < SD - 1 ? MP - 1 - I : SD - 1;
+        static_assert(SD * kLoads <= 63, "the counter holds every load in flight");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter * kLoads) : "memory");
+    }
+    // the reads of a slot are complete
+    __device__ __forceinline__ void release() const { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+};
+
 // ------------------------------------------------------------ TENO kernel
 // 64 cells per 256-thread block, 4 lanes (a quad) per cell.
 // Phase A: quad lane s owns stencil s: stencil-major loads of ids, areas and
@@ -174,7 +249,9 @@ __device__ inline double legendre_le2(int p, double x) {
 // the face-point basis values are recomputed from the cell's node
 // coordinates with the precompute's operations in its order, so they equal
 // the table bit for bit, and the per-cell face basis is not read.
-template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, bool CT = false, bool DV = false>
+// SD: stream depth (plain pass, unrolled members, odd KP): the member tables
+// come through LDS (see member_stream), in SD slots per wave from sh_net on.
+template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, bool CT = false, bool DV = false, int SD = 0>
 __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const double* __restrict__ U,
                                            double* __restrict__ fs, uint8_t* __restrict__ dec, const Physics& ph,
                                            uint32_t lb, double2* sh_u, unsigned char* sh_net) {
@@ -184,6 +261,14 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     constexpr bool kFullOnly = GM == 5;
     const uint32_t N = g.N;
     if (lb * 64u >= N) return;  // whole block past the end (uniform)
+    using Stream = MemberStream<KP, MP, IdxT, SD>;
+    [[maybe_unused]] Stream stream;
+    if constexpr (SD > 0) {
+        static_assert(GM == 0 && MP > 0 && !CT, "streamed tables: the plain pass at a compiled stencil size");
+        stream.init(t, lb, sh_net);
+#pragma unroll
+        for (int i = 0; i < (SD < MP ? SD : MP); ++i) stream.issue();
+    }
     if constexpr (kFullOnly) {
         // the 4 wave marks of the block as one word (uniform)
         if (reinterpret_cast<const uint32_t*>(t.blk_mixed)[lb] == 0u) return;
@@ -282,9 +367,16 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     // per 4 x 4 transpose instead of the DPP form's selects and moves. A
     // wave reads only its own lanes' entries, and a wave's LDS accesses run
     // in order, so wave-scope fences (compiler ordering) suffice.
-    constexpr bool kLdsX = (GM == 0 || GM == 4 || GM == 5) && TILE == 256;
-    constexpr int kXs = 258;
-    __shared__ double xbuf[kLdsX ? 4 * kXs : 1];
+    // A streamed pass takes them through its own wave's slots, which hold
+    // nothing any more then.
+    constexpr bool kLdsX = ((GM == 0 || GM == 4 || GM == 5) && TILE == 256) || SD > 0;
+    constexpr int kXs = SD > 0 ? 66 : 258;
+    __shared__ double xbuf_block[kLdsX && SD == 0 ? 4 * kXs : 1];
+    double* xbuf = xbuf_block;
+    if constexpr (SD > 0) {
+        static_assert(4 * kXs * 8 <= SD * Stream::kSlot, "the exchange fits the wave's slots");
+        xbuf = reinterpret_cast<double*>(stream.base);
+    }
     auto wave_sync = []() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -293,7 +385,7 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     // out[j] = x[q] of quad lane j
     auto exchange = [&](const double* x, double* out) {
         if constexpr (kLdsX) {
-            const uint32_t tid = threadIdx.x, base = tid & ~3u;
+            const uint32_t tid = SD > 0 ? threadIdx.x & 63u : threadIdx.x, base = tid & ~3u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) xbuf[i * kXs + tid] = x[i];
             wave_sync();
@@ -384,8 +476,47 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
 #pragma unroll
             for (int v = 0; v < 4; ++v) a[k][v] = 0.0;
         double w[4] = {0.0, 0.0, 0.0, 0.0};
+        if constexpr (SD > 0) {
+            // every lane runs along (a lane without a stencil reads table
+            // entries of no meaning and the tile's first cell) and is cleared after
+            each_index<MP>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                stream.template wait<i>();
+                const unsigned char* m = stream.slot(i);
+                const int lane = threadIdx.x & 63;
+                const uint32_t p = reinterpret_cast<const IdxT*>(m + Stream::kRows * 512)[lane];
+                const uint32_t pos = active ? p : 0u;
+                const double* Am = reinterpret_cast<const double*>(m) + lane;
+                const double tt = Am[KP * 64];
+                const double2 u01 = sh_u[2 * pos], u23 = sh_u[2 * pos + 1];
+                const double b[4] = {tt * (u01.x - uc.v[0]), tt * (u01.y - uc.v[1]), tt * (u23.x - uc.v[2]),
+                                     tt * (u23.y - uc.v[3])};
+#pragma unroll
+                for (int k = 0; k < KP; ++k) {
+                    const double Ak = Am[k * 64];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        a[k][v] = a[k][v] + Ak * b[v];
+                        // summed here: sunk to the sums' uses the products' operands would all stay live
+                        asm volatile("" : "+v"(a[k][v]));
+                    }
+                }
+                if constexpr (i + SD < MP) {
+                    stream.release();
+                    stream.issue();
+                }
+            });
+            if (!active) {
+#pragma unroll
+                for (int k = 0; k < KP; ++k)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) a[k][v] = 0.0;
+            }
+        }
+        [[maybe_unused]] const auto* oi = (const __attribute__((address_space(4))) double*)t.oi;
         if (active) {
-            if constexpr (MP > 0) {
+            if constexpr (SD > 0) {
+            } else if constexpr (MP > 0) {
 #pragma unroll
                 for (int i = 0; i < MP; ++i) member(i, a);
             } else {
@@ -398,7 +529,7 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
                 for (int k = 0; k < KP; ++k) {
                     double oia = 0.0;
 #pragma unroll
-                    for (int j = 0; j < KP; ++j) oia = oia + t.OI[k * KP + j] * a[j][v];
+                    for (int j = 0; j < KP; ++j) oia = oia + (SD > 0 ? oi[k * KP + j] : t.OI[k * KP + j]) * a[j][v];
                     si = si + a[k][v] * oia;
                 }
                 w[v] = 1.0 / pow6_cr(si + 1.0e-12);
@@ -572,6 +703,18 @@ void teno_kernel(Geom g, Teno t, const double* __restrict__ U,
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     teno_block<KP, MP, FQ, IdxT, TILE, GM, CT, DV>(g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem),
                                                    teno_smem + TILE * 32);
+}
+
+// the plain pass with streamed member tables: dynamic LDS holds the tile
+// (tile_bytes) and the waves' slots
+template <int KP, int MP, int FQ, typename IdxT, int SD, int OCC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
+void teno_stream_kernel(Geom g, Teno t, const double* __restrict__ U, double* __restrict__ fs,
+                        uint8_t* __restrict__ dec, Physics ph, uint32_t tile_bytes, uint32_t blocks_per_xcd) {
+    extern __shared__ __align__(16) unsigned char teno_smem[];
+    const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
+    teno_block<KP, MP, FQ, IdxT, 0, 0, false, false, SD>(g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem),
+                                                      teno_smem + tile_bytes);
 }
 
 // case of global block gb: the last case whose first block is <= gb
@@ -1394,6 +1537,27 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         }
         return hipGetLastError();
     }
+    if (FQ == 6 && Kp == 9 && Mp == 19 && !t.gate) {
+        // plain p = 3 at the default stencil size: streamed member tables.
+        // 36 accumulators a lane leave the plain loop 3 waves per SIMD that
+        // wait on memory 82% of the time (or 4 that spill); with two members
+        // ahead in LDS (51 KB a block, 3 blocks a CU) the pass runs at 95% of
+        // what the tables' bytes allow: 524,288 cells 1,124 -> 695 us, 80,000
+        // 205 -> 118. Three members ahead (2 blocks a CU) 720, 4 waves 760.
+        // At p = 2, where the plain loop keeps 4 waves busy, streaming gains
+        // nothing (1,048,576 cells: 1,141 against 1,127 us) and the smallest
+        // meshes lose 3 us.
+        constexpr int kDepth = 2;
+        const uint32_t tile = t.tile_max * 32;
+        const size_t slots = 4 * kDepth * (10 * 512 + 64 * (small ? 1 : 2));
+        if (small)
+            hipLaunchKernelGGL((teno_stream_kernel<9, 19, 6, uint8_t, kDepth, 3>), grid, block, tile + slots, stream, g,
+                               t, U, fs, dec, ph, tile, per_xcd);
+        else
+            hipLaunchKernelGGL((teno_stream_kernel<9, 19, 6, uint16_t, kDepth, 3>), grid, block, tile + slots, stream,
+                               g, t, U, fs, dec, ph, tile, per_xcd);
+        return hipGetLastError();
+    }
     // the default stencil size (factor 2: M = 2K) is compiled with the member
     // loop unrolled, and at p = 2 in three occupancy targets; other sizes
     // take the runtime loop
@@ -1439,17 +1603,9 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         case 2: MLR_TENO_G(2, 0, 6, 0); break;
         case 5: MLR_TENO(5, 0, 6); break;
         case 9:
-            if (Mp == 19 && !t.gate && (occ == 4 || occ == 5)) {  // plain p = 3 at an occupancy target
-                if (small && occ == 4) MLR_TENO_S(9, 19, 6, 0, 4);
-                else if (small) MLR_TENO_S(9, 19, 6, 0, 5);
-                else if (occ == 4)
-                    hipLaunchKernelGGL((teno_kernel<9, 19, 6, uint16_t, 1024, 0, 4>), grid, block, 1024 * 32, stream,
-                                       g, t, U, fs, dec, ph, per_xcd);
-                else
-                    hipLaunchKernelGGL((teno_kernel<9, 19, 6, uint16_t, 1024, 0, 5>), grid, block, 1024 * 32, stream,
-                                       g, t, U, fs, dec, ph, per_xcd);
-            } else if (Mp == 19) {
-                MLR_TENO(9, 19, 6);
+            if (Mp == 19) {
+                if (gate_reuse) MLR_TENO_G(9, 19, 6, 2);
+                else MLR_TENO_G(9, 19, 6, 1);
             } else {
                 MLR_TENO(9, 0, 6);
             }

@@ -423,6 +423,10 @@ void Solver::upload() {
             up(A_, L_.st_A);
         }
         up(fbasis_, L_.fbasis);
+        std::vector<double> oi;
+        for (int i = 1; i < L_.K; ++i)
+            for (int j = 1; j < L_.K; ++j) oi.push_back(L_.OI[(size_t)i * L_.K + j]);
+        up(oi_, oi);
         if (L_.S == 3 && L_.Q == 1 && L_.K == 6 && L_.M == 12 && !L_.st_loc8.empty() &&
             L_.tspec.basis == BasisType::Legendre && L_.qface_pts.size() == 1) {
             // the cells' node coordinates, for the plain TENO pass's derived face basis
@@ -518,10 +522,12 @@ dev::Teno Solver::teno() const {
     t.loc16 = loc16_;
     t.blk_off = blk_off_;
     t.blk_ids = blk_ids_;
+    t.tile_max = L_.tile_max;
     t.ta = ta_;
     t.A = A_;
     t.fbasis = fbasis_;
     const int Kp = L_.K - 1;
+    t.oi = oi_;
     for (int i = 0; i < Kp; ++i)
         for (int j = 0; j < Kp; ++j) t.OI[i * Kp + j] = L_.OI[(size_t)(i + 1) * L_.K + (j + 1)];
     t.gamma = ph_.gamma;
@@ -960,17 +966,15 @@ void Solver::autotune() {
             HIP_OK(hipMemcpyAsync(saved, gated_, gated_slots_ * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream_));
         }
         // occupancy targets: 5 and 6 waves per SIMD for the p = 2 kernels
-        // (not for split gated passes), 4 and 5 for plain p = 3 with the
-        // default stencil size; the compiler's own choice (0) everywhere.
+        // (not for split gated passes); the compiler's own choice (0) everywhere.
         // The plain p = 2 pass also tries its derived face basis at 0, 4 and 5.
         const bool occ_tunable = L_.K == 6 && L_.M == 12 && fq == 3 && loc8_ != nullptr && !(gate_ && gate_split_);
-        const bool occ_p3 = L_.K == 10 && L_.M == 20 && fq == 6 && !gate_;
         const bool derivable = cvert_ != nullptr && !gate_ && !compact_;
         bt = 1e30f;
         for (int fb : {0, 1}) {
             if (fb == 1 && !derivable) continue;
             for (int occ : {0, 4, 5, 6}) {
-                if (fb == 0 && occ != 0 && !(occ_tunable && occ >= 5) && !(occ_p3 && occ <= 5)) continue;
+                if (fb == 0 && occ != 0 && !(occ_tunable && occ >= 5)) continue;
                 if (fb == 1 && occ == 6) continue;
                 tune_.teno_face_basis = fb;
                 const float t = timed([&] {

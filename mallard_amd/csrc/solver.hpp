@@ -244,6 +244,7 @@ private:
     uint32_t* blk_off_ = nullptr;
     int32_t* blk_ids_ = nullptr;
     double *ta_ = nullptr, *A_ = nullptr, *fbasis_ = nullptr;
+    double* oi_ = nullptr;  // oscillation indicator, (K-1) x (K-1)
     bool compact_ = false;
     double* fbc_ = nullptr;  // compact tables: basis values per reference edge
     // derived face basis: [N][6] node coordinates of each cell (null where
