@@ -1053,6 +1053,7 @@ __device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, co
     const uint32_t last = N - first < bs ? N : first + bs;
     const uint32_t f0 = g.face_off[first >> 6], nf = g.face_off[(last + 63u) >> 6] - f0;
     for (uint32_t i = threadIdx.x; i < nf; i += blockDim.x) {
+        if (a.parts != 3 && !(a.parts & (g.face_meta[f0 + i] & kFaceBoundary ? 2 : 1))) continue;
         double F[4];
         face_flux<RS, PP, VISC>(g, a, ph, f0 + i, F);
 #pragma unroll

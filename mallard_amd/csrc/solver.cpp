@@ -298,8 +298,11 @@ void Solver::setup(Mesh&& mesh) {
     // shapes of contexts that are not autotuned (programs that only call the
     // residual): HLLC flux pass of 8,192 triangles 8.9 us with 128-cell
     // blocks, 15.8 with 256; of 524,288 52 us with either; of 2,097,152 190
-    // against 174
+    // against 174. The derived face basis pays where the pass is bound by
+    // bytes: 262,088 cells 4 us of 162, 8,388,608 cells 166 us of 4,671; below
+    // it costs up to 1.6 us
     if (!tuned_ && L_.N <= (1u << 18)) tune_.flux_block = 128;
+    if (!tuned_ && L_.N > (1u << 18) && cvert_) tune_.teno_face_basis = 1;
     t_ = 0.0;
     step_ = 0;
     wall0_ = wall_seconds();
