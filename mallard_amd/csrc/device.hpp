@@ -128,6 +128,9 @@ struct Teno {
     // the ungated cells); one byte per wave slot (block * 4 + wave), 1 when
     // the wave holds a valid cell the network did not gate
     uint8_t* blk_mixed;
+    // split passes of one solver: the blocks blk_mixed marks, listed after
+    // each evaluation ([0] their number, then the block indices in order)
+    uint32_t* mixed_list;
     // compact tables (corrected weighting, one face point per face): A holds
     // A+ times the member areas (ta unused) and the face-point basis values
     // come from fbc[e][K-1], one row per reference-triangle edge e (the
@@ -230,6 +233,8 @@ hipError_t spectral_radius(const Geom& g, const double* Un, const double* prims,
 // dt = cfl / (max over the n_blk block maxima), or fixed_dt when > 0
 hipError_t finalize_dt(const unsigned long long* lam_blk, uint32_t n_blk, double cfl, double fixed_dt, double* dt,
                        double* dt_hist, int64_t hist_cap, int64_t* step, hipStream_t stream);
+// the marked blocks of a split gated pass, from Teno::blk_mixed into Teno::mixed_list
+hipError_t list_mixed(const Teno& t, uint32_t N, hipStream_t stream);
 hipError_t copy_state(const double* src, double* dst, uint32_t N, hipStream_t stream);
 // viscous runs: per cell (u, v, T, mu) and least-squares gradients of u, v, T
 // of the state U (bs cells per block)

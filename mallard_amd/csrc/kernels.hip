@@ -261,17 +261,25 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     constexpr bool kFullOnly = GM == 5;
     const uint32_t N = g.N;
     if (lb * 64u >= N) return;  // whole block past the end (uniform)
+    // the block's wave marks as one word (uniform)
+    [[maybe_unused]] uint32_t marks = 0xFFFFFFFFu;
+    if constexpr (kFullOnly) {
+        marks = reinterpret_cast<const uint32_t*>(t.blk_mixed)[lb];
+        if (marks == 0u) return;
+    }
     using Stream = MemberStream<KP, MP, IdxT, SD>;
     [[maybe_unused]] Stream stream;
+    [[maybe_unused]] bool streams = true;  // (uniform in a wave)
     if constexpr (SD > 0) {
-        static_assert(GM == 0 && MP > 0 && !CT, "streamed tables: the plain pass at a compiled stencil size");
-        stream.init(t, lb, sh_net);
+        // every lane of a wave takes part in its loads, so a streamed pass
+        // runs whole waves: those that hold a cell it reconstructs
+        static_assert((GM == 0 || GM == 5) && MP > 0 && !CT, "streamed tables: a full pass at a compiled stencil size");
+        if (kFullOnly) streams = ((marks >> (8 * __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)))) & 0xFFu) != 0u;
+        if (streams) {
+            stream.init(t, lb, sh_net);
 #pragma unroll
-        for (int i = 0; i < (SD < MP ? SD : MP); ++i) stream.issue();
-    }
-    if constexpr (kFullOnly) {
-        // the 4 wave marks of the block as one word (uniform)
-        if (reinterpret_cast<const uint32_t*>(t.blk_mixed)[lb] == 0u) return;
+            for (int i = 0; i < (SD < MP ? SD : MP); ++i) stream.issue();
+        }
     }
     {
         const uint32_t t0 = t.blk_off[lb], nloc = t.blk_off[lb + 1] - t0;
@@ -281,6 +289,7 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
         if (kEval && t.gate) ind::stage_net(t.net, sh_net);  // the network, once per block
     }
     __syncthreads();
+    if (SD > 0 && !streams) return;
     const IdxT* __restrict__ loc = sizeof(IdxT) == 1 ? reinterpret_cast<const IdxT*>(t.loc8)
                                                      : reinterpret_cast<const IdxT*>(t.loc16);
     const int q = threadIdx.x & 3;
@@ -645,7 +654,9 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
         for (int fq = 0; fq < FQ; ++fq) f[fq] = ucv;
     };
 
-    if constexpr (kFullOnly) {
+    if constexpr (SD > 0) {
+        full_teno();  // of gated cells too: nothing of theirs is stored
+    } else if constexpr (kFullOnly) {
         if (smooth) skip();
         else full_teno();
     } else if (GM != 0 && t.gate && __all(smooth || !valid)) {
@@ -703,6 +714,70 @@ void teno_kernel(Geom g, Teno t, const double* __restrict__ U,
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     teno_block<KP, MP, FQ, IdxT, TILE, GM, CT, DV>(g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem),
                                                    teno_smem + TILE * 32);
+}
+
+// The ungated cells of a split gated pass (mode 5), block by block from the
+// list of marked blocks. Few blocks are marked (400 of 8,192 at 524,288
+// cells), so the pass is one block's chain, most of it waiting for tables no
+// cache holds: streaming them two members ahead takes 43 us to 24. The list
+// keeps the other blocks from being started: with a grid over every block
+// 64 us streamed and 34 not; at 8,388,608 cells 47 us against 123 for the
+// grid without streaming. Four members ahead and two blocks a CU: the same.
+constexpr uint32_t kUngatedBlocks = 2048;  // two of the chip's fill; each walks its share of the list
+constexpr int kUngatedDepth = 2;
+template <bool CT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void teno_ungated_kernel(Geom g, Teno t, const double* __restrict__ U, double* __restrict__ fs,
+                         uint8_t* __restrict__ dec, Physics ph) {
+    extern __shared__ __align__(16) unsigned char teno_smem[];
+    // each XCD takes one contiguous eighth of the list
+    const uint32_t count = t.mixed_list[0], chunk = (count + 7u) >> 3, lo = (blockIdx.x & 7u) * chunk;
+    const uint32_t hi = lo + chunk < count ? lo + chunk : count;
+    for (uint32_t k = lo + (blockIdx.x >> 3); k < hi; k += gridDim.x >> 3) {
+        teno_block<5, 11, 3, uint8_t, 256, 5, CT, false, CT ? 0 : kUngatedDepth>(
+            g, t, U, fs, dec, ph, t.mixed_list[1 + k], reinterpret_cast<double2*>(teno_smem), teno_smem + 256 * 32);
+        __syncthreads();  // the next block's tile reuses the LDS
+    }
+}
+
+// The marked blocks in ascending order: one block scans 4,096 marks a round.
+__global__ __launch_bounds__(1024) void list_mixed_kernel(const uint32_t* __restrict__ marks, uint32_t n,
+                                                          uint32_t* __restrict__ list) {
+    __shared__ uint32_t wave_sum[2][16];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    uint32_t total = 0;
+    auto load = [&](uint32_t i, uint32_t (&m)[4]) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) m[k] = i + k < n ? marks[i + k] : 0u;
+    };
+    uint32_t m[4], next[4];
+    load(4 * threadIdx.x, m);
+    for (uint32_t base = 0, round = 0; base < n; base += 4096, round ^= 1u) {
+        load(base + 4096 + 4 * threadIdx.x, next);
+        uint32_t mine = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mine += m[k] ? 1u : 0u;
+        uint32_t incl = mine;
+        for (uint32_t off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(incl, off);
+            if (lane >= off) incl += o;
+        }
+        if (lane == 63) wave_sum[round][w] = incl;
+        __syncthreads();
+        uint32_t at = total + incl - mine, sum = 0;
+        for (uint32_t k = 0; k < 16; ++k) {
+            const uint32_t s = wave_sum[round][k];
+            if (k < w) at += s;
+            sum += s;
+        }
+        total += sum;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            if (m[k]) list[1 + at++] = base + 4 * threadIdx.x + k;
+            m[k] = next[k];
+        }
+    }
+    if (threadIdx.x == 0) list[0] = total;
 }
 
 // the plain pass with streamed member tables: dynamic LDS holds the tile
@@ -1456,6 +1531,12 @@ __global__ void probe_kernel(const double* x, const double* y, double* out, int 
 
 }  // namespace
 
+hipError_t list_mixed(const Teno& t, uint32_t N, hipStream_t stream) {
+    hipLaunchKernelGGL(list_mixed_kernel, dim3(1), dim3(1024), 0, stream,
+                       reinterpret_cast<const uint32_t*>(t.blk_mixed), (N + 63) / 64, t.mixed_list);
+    return hipGetLastError();
+}
+
 hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs, uint8_t* dec,
                       const Physics& ph, int occ, int gate_reuse, hipStream_t stream) {
     const int Kp = t.K - 1, Mp = t.M - 1;
@@ -1487,6 +1568,18 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         else MLR_TENO_G(KP, MP, FQV, 1);                   \
     } while (0)
     if (t.gate && Mp < ind::kMembers - 1) return hipErrorInvalidValue;
+    // the second part of a split gated pass: the marked blocks, listed anew
+    // after each evaluation
+    auto ungated = [&](bool compact) {
+        if (!gate_reuse)
+            if (const hipError_t e = list_mixed(t, g.N, stream); e != hipSuccess) return e;
+        const dim3 ug(8 * per_xcd < kUngatedBlocks ? 8 * per_xcd : kUngatedBlocks);
+        if (compact)
+            hipLaunchKernelGGL((teno_ungated_kernel<true>), ug, block, 256 * 32, stream, g, t, U, fs, dec, ph);
+        else
+            hipLaunchKernelGGL((teno_ungated_kernel<false>), ug, block, 256 * 32 + 4 * kUngatedDepth * (6 * 512 + 64), stream, g, t, U, fs, dec, ph);
+        return hipGetLastError();
+    };
     if (t.derived) {
         // derived face basis: plain TENO at p = 2 with the default stencil
         // size and 8-bit tile positions
@@ -1517,8 +1610,7 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
             if (gate_reuse) MLR_TENO_S(5, 11, 3, 4, 0);
             else MLR_TENO_S(5, 11, 3, 3, 0);
             if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-            hipLaunchKernelGGL((teno_kernel<5, 11, 3, uint8_t, 256, 5, 0, true>), grid, block, lds, stream, g, t, U,
-                               fs, dec, ph, per_xcd);
+            return ungated(true);
         } else if (!t.gate) {
             if (occ == 5)
                 hipLaunchKernelGGL((teno_kernel<5, 11, 3, uint8_t, 256, 0, 5, true>), grid, block, lds, stream, g, t,
@@ -1576,8 +1668,7 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
                 if (gate_reuse) MLR_TENO_S(5, 11, 3, 4, 0);
                 else MLR_TENO_S(5, 11, 3, 3, 6);
                 if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-                hipLaunchKernelGGL((teno_kernel<5, 11, 3, uint8_t, 256, 5, 0>), grid, block, 256 * 32, stream, g, t, U,
-                                   fs, dec, ph, per_xcd);
+                return ungated(false);
             } else if (Mp == 11 && small) {
                 const int gm = !t.gate ? 0 : (gate_reuse ? 2 : 1);
 #define MLR_TENO_O(GMV)                                       \

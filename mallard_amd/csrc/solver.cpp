@@ -538,6 +538,7 @@ dev::Teno Solver::teno() const {
     t.gate_dec = gate_dec_;
     t.lin = lin_;
     t.blk_mixed = (gate_ && gate_split_) ? blk_mixed_ : nullptr;
+    t.mixed_list = mixed_list_;
     t.compact = compact_ ? 1 : 0;
     t.fbc = fbc_;
     t.gate = gate_ ? 1 : 0;
@@ -640,6 +641,13 @@ void Solver::set_indicator(const float* params, double threshold) {
         HIP_OK(hipMalloc((void**)&blk_mixed_, nmix));
         allocs_.push_back(blk_mixed_);
         HIP_OK(hipMemset(blk_mixed_, 1, nmix));
+        HIP_OK(hipMalloc((void**)&mixed_list_, nmix + sizeof(uint32_t)));
+        allocs_.push_back(mixed_list_);
+        HIP_OK(hipStreamSynchronize(nullptr));  // stream_ does not wait for the fills
+        dev::Teno marks{};
+        marks.blk_mixed = blk_mixed_;
+        marks.mixed_list = mixed_list_;
+        HIP_OK(dev::list_mixed(marks, L_.N, stream_));
         // the central stencils' linear operators the gated cells use
         const size_t nl = L_.n_pad() * (size_t)L_.S * L_.Q * (size_t)(L_.M - 1);
         HIP_OK(hipMalloc((void**)&lin_, nl * sizeof(double)));

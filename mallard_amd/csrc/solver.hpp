@@ -265,6 +265,7 @@ private:
     double* lin_ = nullptr;        // central stencils' linear operators (gated cells)
     bool gate_per_stage_ = false;
     bool gate_split_ = true;
+    uint32_t* mixed_list_ = nullptr;  // split passes: the blocks that hold ungated cells
     uint8_t* blk_mixed_ = nullptr;  // split passes: per wave slot, 1 when it holds an ungated cell
     size_t gated_slots_ = 0;
     void* net_buf_ = nullptr;
