@@ -38,12 +38,27 @@ constexpr uint32_t kFaceSlot1Shift = 2, kFaceBoundary = 1u << 4, kFaceBcShift = 
 // the face (bit 11 + slot) and whether it is a boundary face (bit 15 + slot).
 constexpr uint32_t kSumCountShift = 8, kSumSideShift = 11, kSumBoundaryShift = 15;
 
+// The ratio of specific heats and the quotients of it that the Riemann
+// solvers use (make_gas): (g - 1)/(2 g), its reciprocal, (g + 1)/(2 g),
+// 2/(g + 1) and (g - 1)/(g + 1)
+struct Gas {
+    double g, z, iz, shock, ta, tb;
+};
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline Gas make_gas(double g) {
+    const double z = (g - 1.0) / (2.0 * g);
+    return Gas{g, z, 1.0 / z, (g + 1.0) / (2.0 * g), 2.0 / (g + 1.0), (g - 1.0) / (g + 1.0)};
+}
+
 struct Physics {
     double gamma, R, cp, cv, p_min, p_max;
     // Navier-Stokes: viscous != 0 adds the viscous fluxes; Sutherland law
     // mu = mu_ref (T/T_mu)^1.5 (T_mu + S)/(T + S) (constant mu_ref when S < 0)
     int32_t viscous;
     double mu_ref, T_mu, S_mu, Pr;
+    Gas gas;  // of gamma
 };
 
 struct BCParam {

@@ -33,7 +33,8 @@ __global__ __launch_bounds__(256) void riemann_points_kernel(int guard, int64_t 
     const double* r = R + 6 * i;
     const double ul[2] = {l[1], l[2]}, ur[2] = {r[1], r[2]};
     double f[4];
-    riemann_flux(RS, guard, f, nrm[2 * i], nrm[2 * i + 1], l[0], ul, l[3], l[4], l[5], r[0], ur, r[3], r[4], r[5]);
+    riemann_flux(RS, guard, f, nrm[2 * i], nrm[2 * i + 1], l[0], ul, l[3], make_gas(l[4]), l[5], r[0], ur, r[3],
+                 make_gas(r[4]), r[5]);
 #pragma unroll
     for (int k = 0; k < 4; ++k) F[4 * i + k] = f[k];
 }

@@ -276,6 +276,7 @@ void Solver::setup(Mesh&& mesh) {
     mesh_ = std::move(mesh);
     // physics.cpp:69-73
     ph_.gamma = cfg_.gamma;
+    ph_.gas = dev::make_gas(cfg_.gamma);
     ph_.R = cfg_.p_ref / (cfg_.T_ref * cfg_.rho_ref);
     ph_.cp = ph_.R * cfg_.gamma / (cfg_.gamma - 1.0);
     ph_.cv = ph_.cp / cfg_.gamma;
