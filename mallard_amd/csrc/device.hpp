@@ -180,6 +180,19 @@ enum StageOp : int32_t {
     kRhsOnly = 8,   // rhs <- k
 };
 
+// The time step joined by the first stage's flux pass itself, from the block
+// maxima of the radii (as finalize_dt), with its history entry and counter.
+struct DtJoin {
+    const unsigned long long* lam_blk;
+    uint32_t n_blk;
+    double cfl, fixed_dt;
+    double* dt;
+    double* dt_hist;
+    int64_t hist_cap;
+    int64_t* step;
+};
+constexpr uint32_t kJoinBlocks = 1024;  // most block maxima a flux block joins
+
 struct StageArgs {
     int32_t op;
     int32_t riemann;
@@ -220,6 +233,11 @@ struct BatchStage {
     int32_t op, fo, corrected;
     int32_t in, out;  // BufRole of the stage input and output
     int32_t pp = 0;   // 1: positivity-preserving flux limiter
+    // 1: the pass finds each case's time step (at most kJoinBlocks maxima a
+    // case; cfl, fixed_dt and hist_cap as in DtJoin)
+    int32_t join = 0;
+    double cfl = 0.0, fixed_dt = 0.0;
+    int64_t hist_cap = 0;
 };
 
 // Launch shapes an autotuner picks per mesh. Every choice gives identical
@@ -239,8 +257,10 @@ struct Tune {
 // evaluating the network again (later stages of a step)
 hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs, uint8_t* decisions,
                       const Physics& ph, int occ, int gate_reuse, hipStream_t stream);
-// bs: cells per block
-hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream);
+// bs: cells per block; join: the pass finds the time step (at most kJoinBlocks
+// maxima), else it reads a.dt
+hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream,
+                       const DtJoin* join = nullptr);
 // spectral radii: lam_cell per cell and, per bs-cell block, the bit pattern
 // of the block's largest radius in lam_blk (NaN radii are ignored)
 hipError_t spectral_radius(const Geom& g, const double* Un, const double* prims, const Physics& ph,
@@ -255,20 +275,21 @@ hipError_t copy_state(const double* src, double* dst, uint32_t N, hipStream_t st
 // of the state U (bs cells per block)
 hipError_t viscous_grad(const Geom& g, const double* U, const Physics& ph, double* vp, double* vg, uint32_t bs,
                         hipStream_t stream);
-// Ensemble launchers: `cases` is a device array of n_cases descriptors whose
-// blk_* offsets are prefix sums (flux and spectral blocks of bs cells, TENO
+// Ensemble launchers: `cases` is a device array of n_cases descriptors and
+// block_case the case of each block of the pass (TENO or flux / spectral). The
+// descriptors' blk_* offsets are prefix sums (flux and spectral blocks of bs cells, TENO
 // blocks of 64); every case has the same K, M, face points, tile-position
 // width (small = 8-bit) and Riemann solver. face_max: the largest number of
 // face-list entries of a flux block in any case.
 // gated: some case runs the learned gate (the block stages the network in LDS);
 // split: every case's gate runs split (Teno::blk_mixed set), as teno_faces
 // derived: plain pass with every case's face basis derived (Teno::derived)
-hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, int in_role, int K, int M, int FQ,
+hipError_t teno_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, int in_role, int K, int M, int FQ,
                       bool small, bool gated, int occ, int gate_reuse, bool split, bool derived, const Physics& ph,
                       hipStream_t stream);
-hipError_t flux_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const BatchStage& st, int riemann,
+hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const BatchStage& st, int riemann,
                       const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream);
-hipError_t spectral_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const Physics& ph, uint32_t bs,
+hipError_t spectral_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const Physics& ph, uint32_t bs,
                           hipStream_t stream);
 hipError_t finalize_batch(const CaseBufs* cases, int n_cases, double cfl, double fixed_dt, int64_t hist_cap,
                           uint32_t bs, hipStream_t stream);
@@ -296,7 +317,8 @@ struct PersistentStep {
     StepBarrier* bar;
     long long spin_ticks;  // longest wait at a barrier, device wall-clock ticks
 };
-hipError_t ensemble_step(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
+hipError_t ensemble_step(const CaseBufs* cases, int n_cases, const uint32_t* teno_case, const uint32_t* flux_case,
+                         uint32_t teno_total, uint32_t flux_total,
                          const PersistentStep& ps, int riemann, bool teno, uint32_t face_max, const Physics& ph,
                          hipStream_t stream, int* grid_out);
 hipError_t probe_math(const double* x, const double* y, double* out, int n, int which, hipStream_t stream);

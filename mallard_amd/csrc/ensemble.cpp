@@ -52,6 +52,9 @@ Ensemble::Ensemble(const Config& base, const std::vector<MeshSpec>& meshes) : cf
     for (const auto& c : cases_) derivable_ = derivable_ && c->cvert_ != nullptr;
     hip_ok(hipStreamCreate(&stream_), "hipStreamCreate");
     hip_ok(hipMalloc(&d_cases_, cases_.size() * sizeof(dev::CaseBufs)), "hipMalloc");
+    uint64_t blocks = 0;
+    for (const auto& c : cases_) blocks += (c->L_.N + 63) / 64;
+    hip_ok(hipMalloc((void**)&d_block_case_, 2 * blocks * sizeof(uint32_t)), "hipMalloc");
     upload_table();
 }
 
@@ -60,6 +63,7 @@ Ensemble::~Ensemble() {
     if (graph_) (void)hipGraphDestroy(graph_);
     for (auto& e : prof_) (void)hipEventDestroy(e.second);
     if (d_cases_) (void)hipFree(d_cases_);
+    if (d_block_case_) (void)hipFree(d_block_case_);
     if (d_bar_) (void)hipFree(d_bar_);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
@@ -68,6 +72,12 @@ uint64_t Ensemble::n_cells() const {
     uint64_t n = 0;
     for (const auto& c : cases_) n += c->L_.N;
     return n;
+}
+
+bool Ensemble::joins() const {
+    for (const auto& c : cases_)
+        if ((c->L_.N + tune_.flux_block - 1) / tune_.flux_block > dev::kJoinBlocks) return false;
+    return true;
 }
 
 uint32_t Ensemble::face_max(uint32_t bs) const {
@@ -95,6 +105,14 @@ void Ensemble::upload_table() {
     }
     teno_blocks_ = bt;
     flux_blocks_ = bf;
+    std::vector<uint32_t> of;
+    of.reserve(bt + bf);
+    for (int pass = 0; pass < 2; ++pass)
+        for (uint32_t k = 0; k < (uint32_t)cases_.size(); ++k) {
+            const uint32_t cells = pass == 0 ? 64 : bs;
+            of.insert(of.end(), (cases_[k]->L_.N + cells - 1) / cells, k);
+        }
+    hip_ok(hipMemcpy(d_block_case_, of.data(), of.size() * sizeof(uint32_t), hipMemcpyHostToDevice), "hipMemcpy");
     hip_ok(hipMemcpy(d_cases_, tab.data(), tab.size() * sizeof(dev::CaseBufs), hipMemcpyHostToDevice), "hipMemcpy");
 }
 
@@ -151,7 +169,6 @@ void Ensemble::set_tune(const dev::Tune& t) {
 void Ensemble::autotune() {
     if (persistent_) return;  // the persistent step's shapes are fixed
     drop_graph();
-    const int n = size();
     hipEvent_t e0, e1;
     hip_ok(hipEventCreate(&e0), "hipEventCreate");
     hip_ok(hipEventCreate(&e1), "hipEventCreate");
@@ -170,12 +187,14 @@ void Ensemble::autotune() {
     const int op = cfg_.integrator == Integrator::RK4 ? dev::kRK4_1 : dev::kSSP1;
     const dev::BatchStage st{op, teno_ ? 0 : 1, corrected, dev::kBufUn, dev::kBufUa, cfg_.positivity ? 1 : 0};
     float bt = 1e30f;
+    best.flux_block = 128;
     for (uint32_t bs : {64u, 128u, 256u}) {
+        if (n_cells() <= (1u << 18)) break;  // as Solver::autotune
         tune_.flux_block = tune_.spec_block = bs;
         upload_table();
         const float t = timed([&] {
-            hip_ok(dev::spectral_batch(d_cases_, n, flux_blocks_, ph_, bs, stream_), "spectral_batch");
-            hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
+            hip_ok(dev::spectral_batch(d_cases_, flux_case(), flux_blocks_, ph_, bs, stream_), "spectral_batch");
+            hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
                    "flux_batch");
         });
         if (t < bt) { bt = t; best.flux_block = bs; }
@@ -201,7 +220,7 @@ void Ensemble::autotune() {
                 if (fb == 0 && (occ == 4 || (occ != 0 && !occ_tunable))) continue;
                 if (fb == 1 && occ == 6) continue;
                 const float t = timed([&] {
-                    hip_ok(dev::teno_batch(d_cases_, n, teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
+                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
                                            0, split_, fb == 1, ph_, stream_), "teno_batch");
                 });
                 if (t < bt) { bt = t; best.teno_occ = occ; best.teno_face_basis = fb; }
@@ -212,7 +231,7 @@ void Ensemble::autotune() {
             for (int occ : {0, 5, 6}) {
                 if (occ != 0 && !occ_tunable) continue;
                 const float t = timed([&] {
-                    hip_ok(dev::teno_batch(d_cases_, n, teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
+                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
                                            1, split_, false, ph_, stream_), "teno_batch");
                 });
                 if (t < bt) { bt = t; best.teno_occ_reuse = occ; }
@@ -248,26 +267,33 @@ void Ensemble::mark(int tag) {
 
 void Ensemble::launch_step(bool prof) {
     (void)prof;
-    const int n = size();
     const int64_t cap = cases_[0]->dt_hist_cap_;
     const uint32_t bs = tune_.flux_block;
-    if (cfg_.use_cfl) hip_ok(dev::spectral_batch(d_cases_, n, flux_blocks_, ph_, bs, stream_), "spectral_batch");
-    hip_ok(dev::finalize_batch(d_cases_, n, cfg_.cfl, cfg_.use_cfl ? 0.0 : cfg_.dt, cap, bs, stream_),
-           "finalize_batch");
+    if (cfg_.use_cfl) hip_ok(dev::spectral_batch(d_cases_, flux_case(), flux_blocks_, ph_, bs, stream_), "spectral_batch");
+    const double fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
+    const bool join = joins();  // the first stage's flux pass finds the time steps
+    if (!join)
+        hip_ok(dev::finalize_batch(d_cases_, size(), cfg_.cfl, fixed_dt, cap, bs, stream_), "finalize_batch");
     mark(kStatDtMs);
     const int corrected = (teno_ && cfg_.teno.variant == TenoVariant::Corrected) ? 1 : 0;
     auto stage = [&](int op, int in, int out) {
         if (teno_) {
             const bool first = op == dev::kSSP1 || op == dev::kRK4_1;
             const int reuse = (gated_ && !gate_per_stage_ && !first) ? 1 : 0;
-            hip_ok(dev::teno_batch(d_cases_, n, teno_blocks_, in, K_, M_, FQ_, small_, gated_,
+            hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, in, K_, M_, FQ_, small_, gated_,
                                    reuse ? tune_.teno_occ_reuse : tune_.teno_occ, reuse, split_,
                                    tune_.teno_face_basis == 1 && !gated_, ph_, stream_),
                    "teno_batch");
             mark(kStatTenoMs);
         }
-        const dev::BatchStage st{op, teno_ ? 0 : 1, corrected, in, out, cfg_.positivity ? 1 : 0};
-        hip_ok(dev::flux_batch(d_cases_, n, flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
+        dev::BatchStage st{op, teno_ ? 0 : 1, corrected, in, out, cfg_.positivity ? 1 : 0};
+        if (join && (op == dev::kSSP1 || op == dev::kRK4_1)) {
+            st.join = 1;
+            st.cfl = cfg_.cfl;
+            st.fixed_dt = fixed_dt;
+            st.hist_cap = cap;
+        }
+        hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
                    "flux_batch");
         mark(kStatFluxMs);
     };
@@ -361,7 +387,7 @@ void Ensemble::launch_persistent(long long* clocks) {
     ps.cfl = cfg_.cfl;
     ps.fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
     ps.hist_cap = cases_[0]->dt_hist_cap_;
-    hip_ok(dev::ensemble_step(d_cases_, size(), teno_blocks_, flux_blocks_, ps, (int)cfg_.riemann, teno_,
+    hip_ok(dev::ensemble_step(d_cases_, size(), teno_case(), flux_case(), teno_blocks_, flux_blocks_, ps, (int)cfg_.riemann, teno_,
                               face_max(256), ph_, stream_, &persistent_grid_), "ensemble_step");
 }
 

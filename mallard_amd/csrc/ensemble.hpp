@@ -62,6 +62,7 @@ public:
 
 private:
     void upload_table();
+    bool joins() const;  // every case's time step is joined by the first stage's flux pass
     uint32_t face_max(uint32_t bs) const;  // most face-list entries of a bs-cell flux block in any case
     void launch_step(bool prof);
     void launch_persistent(long long* clocks);
@@ -73,6 +74,10 @@ private:
     Config cfg_;
     std::vector<std::unique_ptr<Solver>> cases_;
     dev::CaseBufs* d_cases_ = nullptr;
+    // the case of each TENO block, then of each flux block (room for 64-cell blocks)
+    uint32_t* d_block_case_ = nullptr;
+    const uint32_t* teno_case() const { return d_block_case_; }
+    const uint32_t* flux_case() const { return d_block_case_ + teno_blocks_; }
     uint32_t teno_blocks_ = 0, flux_blocks_ = 0;
     int K_ = 0, M_ = 0, FQ_ = 0;
     bool small_ = true, teno_ = false, gated_ = false, gate_per_stage_ = false, split_ = false;

@@ -792,17 +792,6 @@ void teno_stream_kernel(Geom g, Teno t, const double* __restrict__ U, double* __
                                                       teno_smem + tile_bytes);
 }
 
-// case of global block gb: the last case whose first block is <= gb
-__device__ inline int case_of_block(const CaseBufs* __restrict__ cs, int n, uint32_t gb, bool flux) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if ((flux ? cs[mid].blk_flux0 : cs[mid].blk_teno0) <= gb) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 __device__ inline const double* case_buf(const CaseBufs& c, int role) {
     return role == kBufUn ? c.Un : (role == kBufUa ? c.Ua : c.Ub);
 }
@@ -812,15 +801,15 @@ __device__ inline double* case_buf_w(const CaseBufs& c, int role) {
 
 // The TENO pass of every case of an ensemble in one launch: the grid covers
 // all cases' 64-cell blocks (XCD-aware order over the whole grid), each
-// block finds its case in the offset table and runs that case's block.
+// block looks its case up and runs that case's block.
 template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, int OCC, bool DV = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC == 0 ? 1 : OCC, OCC == 0 ? 8 : OCC)))
-void teno_batch_kernel(const CaseBufs* __restrict__ cases, int n_cases, int in_role,
+void teno_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __restrict__ teno_case, int in_role,
                                                          uint32_t total, Physics ph, uint32_t blocks_per_xcd) {
     extern __shared__ __align__(16) unsigned char teno_smem[];
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     if (gb >= total) return;
-    const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, false)];
+    const CaseBufs& cs = cases[teno_case[gb]];
     teno_block<KP, MP, FQ, IdxT, TILE, GM, false, DV>(cs.g, cs.t, case_buf(cs, in_role), cs.fs, cs.dec, ph,
                                                       gb - cs.blk_teno0, reinterpret_cast<double2*>(teno_smem),
                                                       teno_smem + TILE * 32);
@@ -1001,7 +990,7 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
 // operator, which has no dt). VISC: the viscous fluxes.
 template <int RS, bool PP, bool VISC>
 __device__ __forceinline__ void face_flux(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t e,
-                                          double* out) {
+                                          [[maybe_unused]] double pdt, double* out) {
     const uint32_t N = g.N, Q = g.Q;
     const uint32_t meta = g.face_meta[e], c0 = g.face_c0[e], c1 = g.face_c1[e];
     const uint32_t s0 = meta & 3u, s1 = (meta >> kFaceSlot1Shift) & 3u, bc = (meta >> kFaceBcShift) & 0xFu;
@@ -1032,7 +1021,7 @@ __device__ __forceinline__ void face_flux(const Geom& g, const StageArgs& a, con
     for (int i = 0; i < 4; i++) F[i] *= 0.5;
     if constexpr (PP) {
         const D4 U0 = ld4(a.Uin, c0), U1 = ld4(a.Uin, c1);
-        const double Sd = (double)g.S, pdt = *a.dt;
+        const double Sd = (double)g.S;
         pp_limit(ph, g.bc, bnd, bc, n0, n1, F, U0.v, Sd * pdt * ar / g.volume[c0], U1.v,
                  Sd * pdt * ar / g.volume[c1]);
     }
@@ -1047,12 +1036,12 @@ __device__ __forceinline__ void face_flux(const Geom& g, const StageArgs& a, con
 }
 
 // The stage's update of cell c with its residual r.
-__device__ __forceinline__ void stage_update(const StageArgs& a, const Physics& ph, uint32_t c, const double* r) {
+__device__ __forceinline__ void stage_update(const StageArgs& a, const Physics& ph, uint32_t c, double dt,
+                                             const double* r) {
     if (a.op == kRhsOnly) {
         st4(a.rhs, c, D4{{r[0], r[1], r[2], r[3]}});
         return;
     }
-    const double dt = *a.dt;
     const D4 un = ld4(a.Un, c);
     D4 out, wa;
     bool final_stage = false;
@@ -1119,22 +1108,66 @@ __device__ __forceinline__ void stage_update(const StageArgs& a, const Physics& 
     }
 }
 
+// JOIN: the pass is a step's first and finds the time step. Every block joins
+// the block maxima of the radii (at most 4 a thread, loaded before the faces
+// and joined at the barrier after them), so the step has no launch of one
+// block for it: 4.5 us of 82 at 8,192 cells, while a block's join adds under
+// 1 us. Above kJoinBlocks maxima one block joins them in its own launch.
+__device__ inline unsigned long long wave_max(unsigned long long m) {
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(m, off);
+        m = o > m ? o : m;
+    }
+    return m;
+}
+
 // lb: flux block of bs cells; sf: LDS for 4 planes of its face-list entries
-template <int RS, bool PP, bool VISC>
+template <int RS, bool PP, bool VISC, bool JOIN>
 __device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t lb,
-                                           uint32_t bs, double* sf) {
+                                           uint32_t bs, double* sf, const DtJoin& jn) {
     const uint32_t N = g.N, first = lb * bs;
     if (first >= N) return;  // whole block past the end (uniform)
     const uint32_t last = N - first < bs ? N : first + bs;
     const uint32_t f0 = g.face_off[first >> 6], nf = g.face_off[(last + 63u) >> 6] - f0;
+    __shared__ unsigned long long sh_max[JOIN ? 4 : 1];
+    unsigned long long m = 0ull;
+    auto share = [&]() {
+        m = wave_max(m);
+        if ((threadIdx.x & 63u) == 0u) sh_max[threadIdx.x >> 6] = m;
+    };
+    auto joined = [&]() {
+        for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) m = sh_max[w] > m ? sh_max[w] : m;
+        return jn.fixed_dt > 0.0 ? jn.fixed_dt : jn.cfl / __longlong_as_double((long long)m);
+    };
+    double dt = 0.0;
+    if constexpr (JOIN) {
+        if (!(jn.fixed_dt > 0.0))
+            for (uint32_t i = threadIdx.x; i < jn.n_blk; i += blockDim.x) m = jn.lam_blk[i] > m ? jn.lam_blk[i] : m;
+        if constexpr (PP) {  // the limiter needs it at the faces
+            share();
+            __syncthreads();
+            dt = joined();
+        }
+    } else if (a.op != kRhsOnly) {
+        dt = *a.dt;
+    }
     for (uint32_t i = threadIdx.x; i < nf; i += blockDim.x) {
         if (a.parts != 3 && !(a.parts & (g.face_meta[f0 + i] & kFaceBoundary ? 2 : 1))) continue;
         double F[4];
-        face_flux<RS, PP, VISC>(g, a, ph, f0 + i, F);
+        face_flux<RS, PP, VISC>(g, a, ph, f0 + i, dt, F);
 #pragma unroll
         for (int k = 0; k < 4; ++k) sf[k * nf + i] = F[k];
     }
+    if constexpr (JOIN && !PP) share();
     __syncthreads();
+    if constexpr (JOIN) {
+        if constexpr (!PP) dt = joined();
+        if (lb == 0 && threadIdx.x == 0) {
+            *jn.dt = dt;
+            if (jn.dt_hist) jn.dt_hist[*jn.step % jn.hist_cap] = dt;
+            *jn.step += 1;
+        }
+    }
     for (uint32_t c = first + threadIdx.x; c < last; c += blockDim.x) {
         const uint32_t slots = g.cell_faces[c], sum = g.cell_sum[c];
         const uint32_t base = g.face_off[c >> 6] - f0, count = (sum >> kSumCountShift) & 0x7u;
@@ -1153,16 +1186,16 @@ __device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, co
         const double vol = g.volume[c];
 #pragma unroll
         for (int k = 0; k < 4; k++) r[k] /= vol;
-        stage_update(a, ph, c, r);
+        stage_update(a, ph, c, dt, r);
     }
 }
 
-template <int RS, bool PP, bool VISC>
+template <int RS, bool PP, bool VISC, bool JOIN>
 __global__ __launch_bounds__(256) void flux_update_kernel(Geom g, StageArgs a, Physics ph, uint32_t bs,
-                                                          uint32_t blocks_per_xcd) {
+                                                          uint32_t blocks_per_xcd, DtJoin jn) {
     extern __shared__ __align__(16) unsigned char flux_smem[];
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    flux_block<RS, PP, VISC>(g, a, ph, lb, bs, reinterpret_cast<double*>(flux_smem));
+    flux_block<RS, PP, VISC, JOIN>(g, a, ph, lb, bs, reinterpret_cast<double*>(flux_smem), jn);
 }
 
 __device__ inline StageArgs case_stage(const CaseBufs& cs, int op, int riemann, int fo, int corrected, int in,
@@ -1187,16 +1220,18 @@ __device__ inline StageArgs case_stage(const CaseBufs& cs, int op, int riemann, 
 
 // The flux + stage update of every case in one launch (blocks of bs cells;
 // the case table's block offsets count blocks of that size).
-template <int RS, bool PP>
-__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases, int n_cases,
+template <int RS, bool PP, bool JOIN>
+__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __restrict__ flux_case,
                                                          BatchStage st, uint32_t total, Physics ph, uint32_t bs,
                                                          uint32_t blocks_per_xcd) {
     extern __shared__ __align__(16) unsigned char flux_smem[];
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     if (gb >= total) return;
-    const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+    const CaseBufs& cs = cases[flux_case[gb]];
     const StageArgs a = case_stage(cs, st.op, RS, st.fo, st.corrected, st.in, st.out);
-    flux_block<RS, PP, false>(cs.g, a, ph, gb - cs.blk_flux0, bs, reinterpret_cast<double*>(flux_smem));
+    DtJoin jn{};
+    if constexpr (JOIN) jn = DtJoin{cs.lam_blk, (cs.g.N + bs - 1) / bs, st.cfl, st.fixed_dt, cs.dt, cs.dt_hist, st.hist_cap, cs.step};
+    flux_block<RS, PP, false, JOIN>(cs.g, a, ph, gb - cs.blk_flux0, bs, reinterpret_cast<double*>(flux_smem), jn);
 }
 
 // ------------------------------------------------------------ dt
@@ -1305,11 +1340,11 @@ __global__ __launch_bounds__(256) void spectral_kernel(Geom g, const double* __r
 
 // spectral radii of every case in one launch (each block inside one case, so
 // the block max goes to that case's maximum)
-__global__ __launch_bounds__(256) void spectral_batch_kernel(const CaseBufs* __restrict__ cases, int n_cases,
+__global__ __launch_bounds__(256) void spectral_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __restrict__ flux_case,
                                                              uint32_t total, Physics ph, uint32_t blocks_per_xcd) {
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     if (gb >= total) return;
-    const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+    const CaseBufs& cs = cases[flux_case[gb]];
     spectral_block(cs.g, cs.Un, cs.prims, ph, cs.lam_cell, cs.lam_blk, gb - cs.blk_flux0);
 }
 
@@ -1390,7 +1425,7 @@ __device__ inline void grid_barrier(StepBarrier* bar, uint32_t n_blocks, long lo
 }
 
 template <int RS, bool TENO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void ensemble_step_kernel(const CaseBufs* __restrict__ cases, int n_cases,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void ensemble_step_kernel(const CaseBufs* __restrict__ cases, int n_cases, const uint32_t* __restrict__ teno_case, const uint32_t* __restrict__ flux_case,
                                                             uint32_t teno_total, uint32_t flux_total,
                                                             PersistentStep ps, Physics ph) {
     extern __shared__ __align__(16) unsigned char step_smem[];
@@ -1409,7 +1444,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     };
     if (ps.use_cfl) {
         each(flux_total, [&](uint32_t gb) {
-            const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+            const CaseBufs& cs = cases[flux_case[gb]];
             spectral_block(cs.g, cs.Un, cs.prims, ph, cs.lam_cell, cs.lam_blk, gb - cs.blk_flux0);
         });
         grid_barrier(ps.bar, G, ps.spin_ticks);
@@ -1425,7 +1460,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     for (int st = 0; st < ps.n_stages; ++st) {
         if constexpr (TENO) {
             each(teno_total, [&](uint32_t gb) {
-                const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, false)];
+                const CaseBufs& cs = cases[teno_case[gb]];
                 teno_block<5, 11, 3, uint8_t, 256, 0>(cs.g, cs.t, case_buf(cs, ps.in[st]), cs.fs, cs.dec, ph,
                                                       gb - cs.blk_teno0, reinterpret_cast<double2*>(step_smem),
                                                       step_smem + 256 * 32);
@@ -1434,10 +1469,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         }
         stamp(3 + 2 * st);
         each(flux_total, [&](uint32_t gb) {
-            const CaseBufs& cs = cases[case_of_block(cases, n_cases, gb, true)];
+            const CaseBufs& cs = cases[flux_case[gb]];
             const StageArgs a = case_stage(cs, ps.op[st], RS, ps.fo, ps.corrected, ps.in[st], ps.out[st]);
-            flux_block<RS, false, false>(cs.g, a, ph, gb - cs.blk_flux0, blockDim.x,
-                                         reinterpret_cast<double*>(step_smem));
+            flux_block<RS, false, false, false>(cs.g, a, ph, gb - cs.blk_flux0, blockDim.x,
+                                                reinterpret_cast<double*>(step_smem), DtJoin{});
         });
         if (st + 1 < ps.n_stages || ps.clocks) grid_barrier(ps.bar, G, ps.spin_ticks);
         stamp(4 + 2 * st);
@@ -1725,21 +1760,30 @@ uint32_t flux_threads(uint32_t bs, uint64_t cells) { return bs < 256 && cells <=
 int face_size(uint32_t bs) { return bs == 64 ? 0 : (bs == 128 ? 1 : 2); }
 }  // namespace
 
-hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream) {
+hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uint32_t bs, hipStream_t stream,
+                       const DtJoin* join) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t nblk = (g.N + bs - 1) / bs, per_xcd = (nblk + 7) / 8;
     const dim3 grid(8 * per_xcd), block(flux_threads(bs, g.N));
     const size_t lds = (size_t)g.face_max[face_size(bs)] * 32;
     const bool pp = a.pp && a.op != kRhsOnly;
     if (a.parts != 3 && a.op != kRhsOnly) return hipErrorInvalidValue;
-#define MLR_FU(RSV)                                                                                        \
-    do {                                                                                                   \
-        if (ph.viscous)                                                                                    \
-            hipLaunchKernelGGL((flux_update_kernel<RSV, false, true>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
-        else if (pp)                                                                                       \
-            hipLaunchKernelGGL((flux_update_kernel<RSV, true, false>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
-        else                                                                                               \
-            hipLaunchKernelGGL((flux_update_kernel<RSV, false, false>), grid, block, lds, stream, g, a, ph, bs, per_xcd); \
+    if (join && (a.op == kRhsOnly || join->n_blk > kJoinBlocks)) return hipErrorInvalidValue;
+    const DtJoin jn = join ? *join : DtJoin{};
+#define MLR_FK(RSV, PPV, VV)                                                                                       \
+    do {                                                                                                           \
+        if (join)                                                                                                  \
+            hipLaunchKernelGGL((flux_update_kernel<RSV, PPV, VV, true>), grid, block, lds, stream, g, a, ph, bs,   \
+                               per_xcd, jn);                                                                       \
+        else                                                                                                       \
+            hipLaunchKernelGGL((flux_update_kernel<RSV, PPV, VV, false>), grid, block, lds, stream, g, a, ph, bs,  \
+                               per_xcd, jn);                                                                       \
+    } while (0)
+#define MLR_FU(RSV)                               \
+    do {                                          \
+        if (ph.viscous) MLR_FK(RSV, false, true); \
+        else if (pp) MLR_FK(RSV, true, false);    \
+        else MLR_FK(RSV, false, false);           \
     } while (0)
     switch (a.riemann) {
     case 0: MLR_FU(0); break;
@@ -1749,6 +1793,7 @@ hipError_t flux_update(const Geom& g, const StageArgs& a, const Physics& ph, uin
     default: return hipErrorInvalidValue;
     }
 #undef MLR_FU
+#undef MLR_FK
     return hipGetLastError();
 }
 
@@ -1768,12 +1813,12 @@ hipError_t finalize_dt(const unsigned long long* lam_blk, uint32_t n_blk, double
     return hipGetLastError();
 }
 
-hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, int in_role, int K, int M, int FQ,
+hipError_t teno_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, int in_role, int K, int M, int FQ,
                       bool small, bool gated, int occ, int gate_reuse, bool split, bool derived, const Physics& ph,
                       hipStream_t stream) {
     const int Kp = K - 1, Mp = M - 1;
     const size_t net_lds = (gated && !gate_reuse) ? ind::kNetInferBytes : 0;
-    if (n_cases < 1 || (FQ != 3 && FQ != 6) || Mp < 1) return hipErrorInvalidValue;
+    if ((FQ != 3 && FQ != 6) || Mp < 1) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
     const dim3 grid(8 * per_xcd), block(256);
     if (derived) {
@@ -1782,13 +1827,13 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
         if (!(FQ == 3 && Kp == 5 && Mp == 11 && small) || gated) return hipErrorInvalidValue;
         if (occ == 4)
             hipLaunchKernelGGL((teno_batch_kernel<5, 11, 3, uint8_t, 256, 0, 4, true>), grid, block, 256 * 32,
-                               stream, cases, n_cases, in_role, total_blocks, ph, per_xcd);
+                               stream, cases, block_case, in_role, total_blocks, ph, per_xcd);
         else if (occ == 5)
             hipLaunchKernelGGL((teno_batch_kernel<5, 11, 3, uint8_t, 256, 0, 5, true>), grid, block, 256 * 32,
-                               stream, cases, n_cases, in_role, total_blocks, ph, per_xcd);
+                               stream, cases, block_case, in_role, total_blocks, ph, per_xcd);
         else if (occ == 0)
             hipLaunchKernelGGL((teno_batch_kernel<5, 11, 3, uint8_t, 256, 0, 0, true>), grid, block, 256 * 32,
-                               stream, cases, n_cases, in_role, total_blocks, ph, per_xcd);
+                               stream, cases, block_case, in_role, total_blocks, ph, per_xcd);
         else
             return hipErrorInvalidValue;
         return hipGetLastError();
@@ -1796,14 +1841,14 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
     if (occ != 0 && occ != 5 && occ != 6) return hipErrorInvalidValue;
 #define MLR_TB_S(KP, MP, FQV, G, O)                                                                             \
     hipLaunchKernelGGL((teno_batch_kernel<KP, MP, FQV, uint8_t, 256, G, O>), grid, block, 256 * 32 + net_lds,   \
-                       stream, cases, n_cases, in_role, total_blocks, ph, per_xcd)
+                       stream, cases, block_case, in_role, total_blocks, ph, per_xcd)
 #define MLR_TB_G(KP, MP, FQV, G)                                                                               \
     do {                                                                                                       \
         if (small)                                                                                             \
             MLR_TB_S(KP, MP, FQV, G, 0);                                                                       \
         else                                                                                                   \
             hipLaunchKernelGGL((teno_batch_kernel<KP, MP, FQV, uint16_t, 1024, G, 0>), grid, block,              \
-                               1024 * 32 + net_lds, stream, cases, n_cases, in_role, total_blocks, ph, per_xcd); \
+                               1024 * 32 + net_lds, stream, cases, block_case, in_role, total_blocks, ph, per_xcd); \
     } while (0)
 #define MLR_TB(KP, MP, FQV)                              \
     do {                                                 \
@@ -1818,7 +1863,7 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
         else MLR_TB_S(5, 11, 3, 3, 6);  // the evaluate pass at 6 waves per SIMD, as teno_faces
         if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         hipLaunchKernelGGL((teno_batch_kernel<5, 11, 3, uint8_t, 256, 5, 0>), grid, block, 256 * 32, stream, cases,
-                           n_cases, in_role, total_blocks, ph, per_xcd);
+                           block_case, in_role, total_blocks, ph, per_xcd);
     } else if (FQ == 3 && Kp == 5 && Mp == 11 && small) {
         const int gm = !gated ? 0 : (gate_reuse ? 2 : 1);
 #define MLR_TB_O(GMV)                                     \
@@ -1842,20 +1887,25 @@ hipError_t teno_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
     return hipGetLastError();
 }
 
-hipError_t flux_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const BatchStage& st, int riemann,
+hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const BatchStage& st, int riemann,
                       const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
     const dim3 grid(8 * per_xcd), block(flux_threads(bs, (uint64_t)total_blocks * bs));
     const size_t lds = (size_t)face_max * 32;
-#define MLR_FB(RSV)                                                                                     \
-    do {                                                                                                \
-        if (st.pp)                                                                                      \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, true>), grid, block, lds, stream, cases, n_cases, st, \
-                               total_blocks, ph, bs, per_xcd);                                          \
-        else                                                                                            \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, false>), grid, block, lds, stream, cases, n_cases, st, \
-                               total_blocks, ph, bs, per_xcd);                                          \
+#define MLR_FBK(RSV, PPV)                                                                                       \
+    do {                                                                                                        \
+        if (st.join)                                                                                            \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, true>), grid, block, lds, stream, cases, block_case, st,  \
+                               total_blocks, ph, bs, per_xcd);                                                  \
+        else                                                                                                    \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, false>), grid, block, lds, stream, cases, block_case, st, \
+                               total_blocks, ph, bs, per_xcd);                                                  \
+    } while (0)
+#define MLR_FB(RSV)                      \
+    do {                                 \
+        if (st.pp) MLR_FBK(RSV, true);   \
+        else MLR_FBK(RSV, false);        \
     } while (0)
     switch (riemann) {
     case 0: MLR_FB(0); break;
@@ -1865,14 +1915,15 @@ hipError_t flux_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks,
     default: return hipErrorInvalidValue;
     }
 #undef MLR_FB
+#undef MLR_FBK
     return hipGetLastError();
 }
 
-hipError_t spectral_batch(const CaseBufs* cases, int n_cases, uint32_t total_blocks, const Physics& ph, uint32_t bs,
+hipError_t spectral_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const Physics& ph, uint32_t bs,
                           hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
-    hipLaunchKernelGGL(spectral_batch_kernel, dim3(8 * per_xcd), dim3(bs), 0, stream, cases, n_cases, total_blocks,
+    hipLaunchKernelGGL(spectral_batch_kernel, dim3(8 * per_xcd), dim3(bs), 0, stream, cases, block_case, total_blocks,
                        ph, per_xcd);
     return hipGetLastError();
 }
@@ -1887,7 +1938,8 @@ hipError_t finalize_batch(const CaseBufs* cases, int n_cases, double cfl, double
 
 namespace {
 template <int RS, bool TENO>
-hipError_t launch_step_persistent(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
+hipError_t launch_step_persistent(const CaseBufs* cases, int n_cases, const uint32_t* teno_case,
+                                  const uint32_t* flux_case, uint32_t teno_total, uint32_t flux_total,
                                   const PersistentStep& ps, uint32_t face_max, const Physics& ph, hipStream_t stream,
                                   int* grid_out) {
     const void* fn = reinterpret_cast<const void*>(&ensemble_step_kernel<RS, TENO>);
@@ -1907,19 +1959,21 @@ hipError_t launch_step_persistent(const CaseBufs* cases, int n_cases, uint32_t t
     uint32_t tt = teno_total, ft = flux_total;
     PersistentStep p = ps;
     Physics h = ph;
-    void* args[] = {&c, &n, &tt, &ft, &p, &h};
+    const uint32_t *tc = teno_case, *fc = flux_case;
+    void* args[] = {&c, &n, &tc, &fc, &tt, &ft, &p, &h};
     return hipLaunchCooperativeKernel(fn, dim3(grid), dim3(256), args, (unsigned)lds, stream);
 }
 }  // namespace
 
-hipError_t ensemble_step(const CaseBufs* cases, int n_cases, uint32_t teno_total, uint32_t flux_total,
+hipError_t ensemble_step(const CaseBufs* cases, int n_cases, const uint32_t* teno_case, const uint32_t* flux_case,
+                         uint32_t teno_total, uint32_t flux_total,
                          const PersistentStep& ps, int riemann, bool teno, uint32_t face_max, const Physics& ph,
                          hipStream_t stream, int* grid_out) {
     if (n_cases < 1 || ps.n_stages < 1 || ps.n_stages > 4) return hipErrorInvalidValue;
 #define MLR_STEP(RSV)                                                                                          \
-    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_total, flux_total, ps, face_max, ph, stream, \
+    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_case, flux_case, teno_total, flux_total, ps, face_max, ph, stream, \
                                                     grid_out)                                                    \
-                : launch_step_persistent<RSV, false>(cases, n_cases, teno_total, flux_total, ps, face_max, ph, stream, \
+                : launch_step_persistent<RSV, false>(cases, n_cases, teno_case, flux_case, teno_total, flux_total, ps, face_max, ph, stream, \
                                                      grid_out)
     switch (riemann) {
     case 0: MLR_STEP(0);

@@ -796,15 +796,15 @@ void Solver::launch_teno(const double* U, bool first_stage) {
     mark(kStatTenoMs);
 }
 
-void Solver::launch_flux(int op, const double* Uin, double* Uout) {
+void Solver::launch_flux(int op, const double* Uin, double* Uout, const dev::DtJoin* join) {
     if (cfg_.viscous) HIP_OK(dev::viscous_grad(geom(), Uin, ph_, vp_, vg_, tune_.flux_block, stream_));
-    HIP_OK(dev::flux_update(geom(), stage(op, Uin, Uout), ph_, tune_.flux_block, stream_));
+    HIP_OK(dev::flux_update(geom(), stage(op, Uin, Uout), ph_, tune_.flux_block, stream_, join));
     mark(kStatFluxMs);
 }
 
-void Solver::stage_pass(int op, const double* Uin, double* Uout) {
+void Solver::stage_pass(int op, const double* Uin, double* Uout, const dev::DtJoin* join) {
     if (L_.teno) launch_teno(Uin, op == dev::kFE || op == dev::kSSP1 || op == dev::kRK4_1 || op == dev::kRhsOnly);
-    launch_flux(op, Uin, Uout);
+    launch_flux(op, Uin, Uout, join);
 }
 
 void Solver::dt_pass(double cfl, double fixed_dt) {
@@ -817,20 +817,29 @@ void Solver::dt_pass(double cfl, double fixed_dt) {
 
 // time_integrator.cpp:57-163 as fused stage passes
 void Solver::launch_step() {
-    dt_pass(cfg_.cfl, cfg_.use_cfl ? 0.0 : cfg_.dt);
+    const double fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
+    const dev::DtJoin jn{lam_blk_, spec_blocks(), cfg_.cfl, fixed_dt, dt_dev_, dt_hist_, dt_hist_cap_, step_dev_};
+    const dev::DtJoin* join = spec_blocks() <= dev::kJoinBlocks ? &jn : nullptr;
+    if (!join) {
+        dt_pass(cfg_.cfl, fixed_dt);
+    } else {  // the first stage's flux pass joins the radii itself
+        if (cfg_.use_cfl)
+            HIP_OK(dev::spectral_radius(geom(), Un_, prims_, ph_, lam_cell_, lam_blk_, tune_.spec_block, stream_));
+        mark(kStatDtMs);
+    }
     switch (cfg_.integrator) {
     case Integrator::FE:
-        stage_pass(dev::kFE, Un_, Ua_);
+        stage_pass(dev::kFE, Un_, Ua_, join);
         HIP_OK(dev::copy_state(Ua_, Un_, L_.N, stream_));
         mark(kStatOtherMs);
         break;
     case Integrator::SSPRK3:
-        stage_pass(dev::kSSP1, Un_, Ua_);
+        stage_pass(dev::kSSP1, Un_, Ua_, join);
         stage_pass(dev::kSSP2, Ua_, Ub_);
         stage_pass(dev::kSSP3, Ub_, Un_);
         break;
     case Integrator::RK4:
-        stage_pass(dev::kRK4_1, Un_, Ua_);
+        stage_pass(dev::kRK4_1, Un_, Ua_, join);
         stage_pass(dev::kRK4_2, Ua_, Ub_);
         stage_pass(dev::kRK4_3, Ub_, Ua_);
         stage_pass(dev::kRK4_4, Ua_, Un_);
@@ -1018,8 +1027,14 @@ void Solver::autotune() {
     // the next dt is computed from); FE's only stage is timed as the residual
     const int op = cfg_.integrator == Integrator::FE ? dev::kRhsOnly
                    : cfg_.integrator == Integrator::RK4 ? dev::kRK4_1 : dev::kSSP1;
+    // up to 262,144 cells 128-cell blocks, untimed: the flux kernel's length is
+    // one thread's chain there, which the (often uniform) initial state does
+    // not show. A Sod step of 1,000 quads 36 us with 128, 42 with 64, 47 with
+    // 256; of 8,192 triangles 81, 81 and 102; of 102,659 quads 71, 74 and 75
     bt = 1e30f;
+    best.flux_block = 128;
     for (uint32_t bs : {64u, 128u, 256u}) {
+        if (L_.N <= (1u << 18)) break;
         const float t = timed([&] {
             if (cfg_.viscous) HIP_OK(dev::viscous_grad(geom(), Un_, ph_, vp_, vg_, bs, stream_));
             HIP_OK(dev::flux_update(geom(), stage(op, Un_, Ua_), ph_, bs, stream_));

@@ -160,7 +160,7 @@ public:
     // kernel-level entry points used by the benchmark's timing harness
     void launch_step();                 // one full step, asynchronously
     void launch_teno(const double* U, bool first_stage = true);  // one TENO face-state pass
-    void launch_flux(int op, const double* Uin, double* Uout);
+    void launch_flux(int op, const double* Uin, double* Uout, const dev::DtJoin* join = nullptr);
     double* d_state() { return Un_; }
     uint64_t device_bytes() const { return dev_bytes_; }  // all device allocations
 
@@ -205,7 +205,7 @@ private:
     dev::Geom geom() const;
     dev::Teno teno() const;
     dev::StageArgs stage(int op, const double* Uin, double* Uout) const;
-    void stage_pass(int op, const double* Uin, double* Uout);
+    void stage_pass(int op, const double* Uin, double* Uout, const dev::DtJoin* join = nullptr);
     void dt_pass(double cfl, double fixed_dt);
     void check_dt_mode() const;
     void mark(int tag);
