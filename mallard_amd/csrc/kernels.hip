@@ -975,15 +975,23 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
 // in the canonical order, divides by the volume and applies the stage's
 // SSP-RK update (no atomics). A flux has the same bits for both cells of its
 // face, so the sums equal a serial run's in the one-thread order.
-// What bounds it: FP64 issue and the chain of divisions, square roots and
-// pows in one flux, then memory. Evaluating a face once per block instead of
-// once per cell takes 1.7 evaluations per cell instead of 3, and reads 58 B
-// of face lists instead of 96 B of slot arrays per cell. HLLC on a flow with
-// waves everywhere (rocprof, one thread per cell and its three faces before):
-// 8,388,608 cells 1,161 -> 895 us, 524,288 72.8 -> 51.9 us, 2,048 26.4 ->
-// 9 us; with the limiter, 73,006 cells 35 -> 16 us; viscous Roe, 99,700 cells
-// 22.8 -> 16 us. Holding the registers (105 for HLLC, 4 waves per SIMD) to 5
-// waves costs time: 8,388,608 cells 957 us, at 6 waves 1,110 us.
+// What bounds it: on a full chip FP64 issue (8,388,608 cells: 2,586 VALU
+// instructions per wave, the SIMDs issuing 77% of the launch, 1.75 GB moved
+// where one thread per cell and its three faces moved 3.07 GB); on small
+// meshes the chain of divisions, square roots and powers in one flux.
+// Evaluating a face once per block instead of once per cell takes 1.7
+// evaluations per cell instead of 3, and reads 58 B of face lists instead of
+// 96 B of slot arrays per cell. HLLC on a flow with waves everywhere (rocprof;
+// one thread per cell -> faces once -> with the leaner powers of
+// riemann.hpp): 8,388,608 cells 1,161 -> 973 -> 871 us on one machine,
+// 524,288 72.8 -> 51.9 -> 49.5 us, 2,048 26.4 -> 9 -> 8.5 us. Faces once
+// alone: with the limiter, 73,006 cells 35 -> 16 us; viscous Roe, 99,700
+// cells 22.8 -> 16 us. Holding the registers (about 100 for HLLC, 4 waves
+// per SIMD) to 5 waves costs time: 8,388,608 cells 957 us against 895, at 6
+// waves 1,110 us. So does pooling the faces that take the two-rarefaction
+// estimate, its powers more than half of a flux's instructions, onto the
+// block's first threads through LDS: 524,288 cells 57.4 us against 50.1, the
+// two barriers and the 28 more registers cost more than the idle lanes.
 // RS: Riemann solver (compile-time, so each instantiation carries one
 // solver's code and registers). PP: the positivity-preserving flux limiter
 // (pp_limit) on every face, for the stage updates (not the residual-only

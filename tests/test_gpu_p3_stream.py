@@ -1,6 +1,7 @@
 """The p = 3 TENO pass with member tables streamed through LDS (runs on an
 MI355X): meshes that end inside, at and after a 64-cell block, 8- and 16-bit
-tile positions, and stencils left empty near the boundary. Rusanov runs the
+tile positions (8 x 300: a tile of 812 cells, more than 64 KB of LDS with the
+ring of members), and stencils left empty near the boundary. Rusanov runs the
 same IEEE operations on both sides: bit-exact against the oracle."""
 import numpy as np
 import pytest
@@ -10,7 +11,7 @@ from test_gpu_parity import pair
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny,pos_bytes", [(6, 5, 1), (8, 4, 1), (11, 6, 1), (40, 37, 2)])
+@pytest.mark.parametrize("nx,ny,pos_bytes", [(6, 5, 1), (8, 4, 1), (11, 6, 1), (40, 37, 2), (8, 300, 2)])
 def test_residual(mlr, oracle, nx, ny, pos_bytes):
     dev, orc, m = pair(mlr, oracle, "cartesian_tri", nx, ny, 0.2, 3, recon="TENO", order=3, teno_variant="corrected",
                        riemann="Rusanov")
