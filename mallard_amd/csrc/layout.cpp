@@ -448,7 +448,7 @@ uint64_t Layout::device_bytes() const {
 }
 
 // Face lists of the flux kernel (see Layout::face_off).
-void build_faces(Layout& L) {
+void build_faces(const Mesh& m, Layout& L) {
     const uint32_t N = L.N, S = L.S, B = Layout::kTileCells;
     const uint32_t nblk = (N + B - 1) / B;
     // slots that contribute to the residual, as a bit mask
@@ -458,13 +458,21 @@ void build_faces(Layout& L) {
         for (uint32_t r = 0; r < nact; ++r) m |= 1u << ((code >> (2 * r)) & 3u);
         return m;
     };
-    // slot l of cell c lists its face unless the lower cell of the block does
-    auto lists = [&](uint32_t c, uint32_t l, uint32_t b) {
+    // slot l of cell c and the neighbour's slot hold the same face, each the
+    // other's: the two cells of the block share one entry. (Mesh arrays may
+    // list a face in one of its cells only, twice in a cell, or between a cell
+    // and itself; such a slot keeps an entry of its own.)
+    auto shared = [&](uint32_t c, uint32_t l) {
         const size_t o = (size_t)l * N + c;
+        const uint32_t other = (uint32_t)L.nb[o], ol = L.info[o] & 3u;
+        return !(L.info[o] & kSlotBoundary) && other != c && other / B == c / B &&
+               m.face_of_cell(L.perm[other], ol) == m.face_of_cell(L.perm[c], l) &&
+               (L.info[(size_t)ol * N + other] & 3u) == l;
+    };
+    // slot l of cell c lists its face unless the lower cell of the block does
+    auto lists = [&](uint32_t c, uint32_t l) {
         if (!((active(c) >> l) & 1u)) return false;
-        if (L.info[o] & kSlotBoundary) return true;
-        const uint32_t other = (uint32_t)L.nb[o];
-        return other / B != b || c < other;
+        return !shared(c, l) || c < (uint32_t)L.nb[(size_t)l * N + c];
     };
     L.face_off.assign(nblk + 1, 0);
 #pragma omp parallel for schedule(static)
@@ -472,7 +480,7 @@ void build_faces(Layout& L) {
         const uint32_t c0 = (uint32_t)b * B, c1 = std::min(N, c0 + B);
         uint32_t n = 0;
         for (uint32_t l = 0; l < S; ++l)
-            for (uint32_t c = c0; c < c1; ++c) n += lists(c, l, (uint32_t)b) ? 1u : 0u;
+            for (uint32_t c = c0; c < c1; ++c) n += lists(c, l) ? 1u : 0u;
         L.face_off[b + 1] = n;
     }
     for (uint32_t b = 0; b < nblk; ++b) L.face_off[b + 1] += L.face_off[b];
@@ -500,7 +508,7 @@ void build_faces(Layout& L) {
                 const uint32_t side = (inf >> 2) & 1u;
                 if (l == 0) L.cell_sum[c] = ((inf >> 8) & 0xFFu) | (((inf >> 16) & 0x7u) << dev::kSumCountShift);
                 L.cell_sum[c] |= (side << (dev::kSumSideShift + l)) | ((bnd ? 1u : 0u) << (dev::kSumBoundaryShift + l));
-                if (!lists(c, l, (uint32_t)b)) continue;
+                if (!lists(c, l)) continue;
                 const uint32_t other = (uint32_t)L.nb[o], nbs = inf & 3u;
                 const size_t e = (size_t)L.face_off[b] + n;
                 L.face_c0[e] = side ? other : c;
@@ -512,7 +520,7 @@ void build_faces(Layout& L) {
                 L.face_ny[e] = L.ny[o];
                 L.face_area[e] = L.area[o];
                 L.cell_faces[c] |= n << (8 * l);
-                if (!bnd && other / B == (uint32_t)b) L.cell_faces[other] |= n << (8 * nbs);
+                if (shared(c, l)) L.cell_faces[other] |= n << (8 * nbs);
                 ++n;
             }
     }
@@ -692,7 +700,7 @@ Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::v
         L.info[j] |= (code << 8) | (nact << 16);
     }
     if (bad) fail("inconsistent cells_of_face / faces_of_cell connectivity");
-    build_faces(L);
+    build_faces(m, L);
 
     if (recon == Recon::FO) {
         L.Q = 1;
