@@ -941,7 +941,11 @@ void Solver::autotune() {
     const int fq = (int)(L_.S * L_.Q);
     const std::vector<int64_t> key = {(int64_t)L_.N, L_.K, L_.M, fq, loc8_ ? 1 : 0, gate_ ? 1 : 0,
                                       (int64_t)cfg_.riemann, L_.teno ? 1 : 0, gate_split_ ? 1 : 0,
-                                      gate_per_stage_ ? 1 : 0, cfg_.viscous ? 1 : 0, compact_ ? 1 : 0};
+                                      gate_per_stage_ ? 1 : 0, cfg_.viscous ? 1 : 0, compact_ ? 1 : 0,
+                                      // what decides whether a shape is accepted (the derived basis) and
+                                      // which kernels are timed
+                                      cvert_ ? 1 : 0, (int64_t)L_.tspec.variant, (int64_t)cfg_.integrator,
+                                      cfg_.positivity ? 1 : 0};
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = cache.find(key);
