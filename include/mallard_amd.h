@@ -185,7 +185,9 @@ int mlr_compact_tables(mlr_ctx* ctx);
  * 0, 4 or 5): 72 fewer bytes per cell to read }. Every choice gives
  * bit-identical results. mlr_autotune times the candidates on the current state and
  * returns the fastest (also run by itself before the first steps, cached per
- * mesh size and numerics); mlr_set_tune pins a choice. */
+ * mesh size and numerics); mlr_set_tune pins a choice. Before either,
+ * mlr_get_tune gives the neutral choice { 0, 256, 256, 0, 0 }, and launches
+ * take the shapes of the mesh size. */
 int mlr_autotune(mlr_ctx* ctx, int32_t* tune);
 int mlr_set_tune(mlr_ctx* ctx, const int32_t* tune);
 int mlr_get_tune(mlr_ctx* ctx, int32_t* tune);

@@ -928,6 +928,7 @@ void Solver::set_tune(const dev::Tune& t) {
     }
     tune_ = t;
     tuned_ = true;
+    shaped_ = true;
     drop_graph();
 }
 

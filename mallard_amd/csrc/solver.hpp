@@ -191,10 +191,12 @@ public:
     // Launch shapes (results are identical for every choice). autotune()
     // times the candidates on the current state and keeps the fastest,
     // cached per mesh size and numerics for the process; it runs by itself
-    // before the first steps unless set_tune() pinned a choice.
+    // before the first steps unless set_tune() pinned a choice. Until one of
+    // the two, tune() gives the neutral choice, which set_tune() takes with
+    // any entry changed; launches follow the mesh size (see setup()).
     void autotune();
     void set_tune(const dev::Tune& t);
-    const dev::Tune& tune() const { return tune_; }
+    dev::Tune tune() const { return shaped_ ? tune_ : dev::Tune{}; }
 
 private:
     void setup(Mesh&& mesh);
@@ -256,6 +258,7 @@ private:
     uint32_t spec_blocks() const { return (L_.N + tune_.spec_block - 1) / tune_.spec_block; }
     dev::Tune tune_{};
     bool tuned_ = false;
+    bool shaped_ = false;  // set_tune() or autotune() has chosen the shapes
     void ensure_tuned() {
         if (!tuned_) autotune();
     }
