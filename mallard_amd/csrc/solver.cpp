@@ -850,7 +850,14 @@ void Solver::launch_step() {
 void Solver::record_step() {
     if (step_exec_) return;
     HIP_OK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    launch_step();
+    try {
+        launch_step();
+    } catch (...) {  // a refused launch must not leave the thread capturing
+        hipGraph_t g = nullptr;
+        (void)hipStreamEndCapture(stream_, &g);
+        if (g) (void)hipGraphDestroy(g);
+        throw;
+    }
     HIP_OK(hipStreamEndCapture(stream_, &step_graph_));
     HIP_OK(hipGraphInstantiate(&step_exec_, step_graph_, nullptr, nullptr, 0));
 }
