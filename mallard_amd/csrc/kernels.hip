@@ -250,8 +250,15 @@ struct MemberStream {
 // coordinates with the precompute's operations in its order, so they equal
 // the table bit for bit, and the per-cell face basis is not read.
 // SD: stream depth (plain pass, unrolled members, odd KP): the member tables
-// come through LDS (see member_stream), in SD slots per wave from sh_net on.
-template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, bool CT = false, bool DV = false, int SD = 0>
+// come through LDS (see MemberStream), in SD slots per wave from sh_net on.
+// TIGHT: the loads of a member are not moved above the member before it. At
+// the 80 registers of 6 waves per SIMD the loads in flight push accumulators
+// to scratch: 2,097,152 cells 1,682 us, 69 registers spilled (1,405 and 34
+// before the face points' limits took the quad's lanes); kept apart 1,254 us
+// and 23. With 96 registers (5 waves) it only takes loads out of flight:
+// 1,115 us, kept apart 1,221.
+template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, bool CT = false, bool DV = false, int SD = 0,
+          bool TIGHT = false>
 __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const double* __restrict__ U,
                                            double* __restrict__ fs, uint8_t* __restrict__ dec, const Physics& ph,
                                            uint32_t lb, double2* sh_u, unsigned char* sh_net) {
@@ -428,6 +435,7 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
 #pragma unroll
             for (int v = 0; v < 4; ++v) a[k][v] = a[k][v] + Ak * b[v];
         }
+        if constexpr (TIGHT) __builtin_amdgcn_sched_barrier(0);
     };
 
     const double ucv = sel4(uc.v, q);  // lane-dependent pick by selects, not a stack array
@@ -702,6 +710,10 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
     }
 }
 
+// TIGHT (see teno_block): the plain pass at the 6-wave target. The gated
+// passes spill less there and the compact tables' pass holds no areas
+constexpr bool keep_members_apart(int gm, int occ, bool ct) { return gm == 0 && occ == 6 && !ct; }
+
 // OCC: waves per SIMD the register allocation targets (0: the compiler's
 // own choice); an autotuner picks it per mesh, results are identical
 template <int KP, int MP, int FQ, typename IdxT, int TILE, int GM, int OCC, bool CT = false, bool DV = false>
@@ -712,8 +724,8 @@ void teno_kernel(Geom g, Teno t, const double* __restrict__ U,
     // dynamic LDS: the tile's states (TILE cells), then the network when gated
     extern __shared__ __align__(16) unsigned char teno_smem[];
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    teno_block<KP, MP, FQ, IdxT, TILE, GM, CT, DV>(g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem),
-                                                   teno_smem + TILE * 32);
+    teno_block<KP, MP, FQ, IdxT, TILE, GM, CT, DV, 0, keep_members_apart(GM, OCC, CT)>(
+        g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem), teno_smem + TILE * 32);
 }
 
 // The ungated cells of a split gated pass (mode 5), block by block from the
@@ -810,9 +822,9 @@ void teno_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __res
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     if (gb >= total) return;
     const CaseBufs& cs = cases[teno_case[gb]];
-    teno_block<KP, MP, FQ, IdxT, TILE, GM, false, DV>(cs.g, cs.t, case_buf(cs, in_role), cs.fs, cs.dec, ph,
-                                                      gb - cs.blk_teno0, reinterpret_cast<double2*>(teno_smem),
-                                                      teno_smem + TILE * 32);
+    teno_block<KP, MP, FQ, IdxT, TILE, GM, false, DV, 0, keep_members_apart(GM, OCC, false)>(
+        cs.g, cs.t, case_buf(cs, in_role), cs.fs, cs.dec, ph, gb - cs.blk_teno0, reinterpret_cast<double2*>(teno_smem),
+        teno_smem + TILE * 32);
 }
 
 // ------------------------------------------------------------ viscous terms
