@@ -429,11 +429,28 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
             for (int v = 0; v < 4; ++v) b[v] = tt * (un.v[v] - uc.v[v]);
         }
         const double* Ai = t.A + teno_a_off(lb, Mp, KP, i, 0, cl, q);
+        if constexpr (MP == 0 && KP == 9) {
+            // a member's 9 rows all loaded before the first is used: left to
+            // itself the compiler saves registers by loading them one at a
+            // time, each waited for. 320,000 cells, 24 members 921 -> 548 us
+            // (882 with the schedule that it chose before the face points'
+            // limits took the quad's lanes), ensembles 834 -> 490. At 5 rows
+            // it loads ahead by itself and this costs 4%.
+            double Ak[KP];
 #pragma unroll
-        for (int k = 0; k < KP; ++k) {
-            const double Ak = Ai[(size_t)k * 256];
+            for (int k = 0; k < KP; ++k) Ak[k] = Ai[(size_t)k * 256];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) a[k][v] = a[k][v] + Ak * b[v];
+            for (int k = 0; k < KP; ++k)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) a[k][v] = a[k][v] + Ak[k] * b[v];
+        } else {
+#pragma unroll
+            for (int k = 0; k < KP; ++k) {
+                const double Ak = Ai[(size_t)k * 256];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) a[k][v] = a[k][v] + Ak * b[v];
+            }
         }
         if constexpr (TIGHT) __builtin_amdgcn_sched_barrier(0);
     };
@@ -1707,8 +1724,8 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         return hipGetLastError();
     }
     // the default stencil size (factor 2: M = 2K) is compiled with the member
-    // loop unrolled, and at p = 2 in three occupancy targets; other sizes
-    // take the runtime loop
+    // loop unrolled up to p = 2, there in three occupancy targets; other sizes
+    // and gated p = 3 take the runtime loop
     if (FQ == 3) {
         switch (Kp) {
         case 2: if (Mp == 5) MLR_TENO_G(2, 5, 3, 0); else MLR_TENO_G(2, 0, 3, 0); break;
@@ -1749,14 +1766,9 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         switch (Kp) {
         case 2: MLR_TENO_G(2, 0, 6, 0); break;
         case 5: MLR_TENO(5, 0, 6); break;
-        case 9:
-            if (Mp == 19) {
-                if (gate_reuse) MLR_TENO_G(9, 19, 6, 2);
-                else MLR_TENO_G(9, 19, 6, 1);
-            } else {
-                MLR_TENO(9, 0, 6);
-            }
-            break;
+        // gated p = 3 at the default stencil size too: the loop unrolled took
+        // 256 registers, 1 wave per SIMD (320,000 cells 1,258 us, 540 here)
+        case 9: MLR_TENO(9, 0, 6); break;
         default: return hipErrorInvalidValue;
         }
     }
