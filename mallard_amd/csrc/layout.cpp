@@ -451,13 +451,6 @@ uint64_t Layout::device_bytes() const {
 void build_faces(const Mesh& m, Layout& L) {
     const uint32_t N = L.N, S = L.S, B = Layout::kTileCells;
     const uint32_t nblk = (N + B - 1) / B;
-    // slots that contribute to the residual, as a bit mask
-    auto active = [&](uint32_t c) {
-        const uint32_t code = (L.info[c] >> 8) & 0xFFu, nact = (L.info[c] >> 16) & 0x7u;
-        uint32_t m = 0;
-        for (uint32_t r = 0; r < nact; ++r) m |= 1u << ((code >> (2 * r)) & 3u);
-        return m;
-    };
     // slot l of cell c and the neighbour's slot hold the same face, each the
     // other's: the two cells of the block share one entry. (Mesh arrays may
     // list a face in one of its cells only, twice in a cell, or between a cell
@@ -469,18 +462,26 @@ void build_faces(const Mesh& m, Layout& L) {
                m.face_of_cell(L.perm[other], ol) == m.face_of_cell(L.perm[c], l) &&
                (L.info[(size_t)ol * N + other] & 3u) == l;
     };
-    // slot l of cell c lists its face unless the lower cell of the block does
-    auto lists = [&](uint32_t c, uint32_t l) {
-        if (!((active(c) >> l) & 1u)) return false;
-        return !shared(c, l) || c < (uint32_t)L.nb[(size_t)l * N + c];
-    };
+    // per cell: bit l where slot l lists its face (it contributes to the
+    // residual, and no lower cell of the block lists it), bit 4 + l where the
+    // entry serves the neighbour too
+    std::vector<uint8_t> own(N);
     L.face_off.assign(nblk + 1, 0);
 #pragma omp parallel for schedule(static)
     for (int64_t b = 0; b < (int64_t)nblk; ++b) {
         const uint32_t c0 = (uint32_t)b * B, c1 = std::min(N, c0 + B);
         uint32_t n = 0;
-        for (uint32_t l = 0; l < S; ++l)
-            for (uint32_t c = c0; c < c1; ++c) n += lists(c, l) ? 1u : 0u;
+        for (uint32_t c = c0; c < c1; ++c) {
+            const uint32_t code = (L.info[c] >> 8) & 0xFFu, nact = (L.info[c] >> 16) & 0x7u;
+            uint32_t mask = 0;
+            for (uint32_t r = 0; r < nact; ++r) {
+                const uint32_t l = (code >> (2 * r)) & 3u;
+                if (!shared(c, l)) mask |= 1u << l;
+                else if (c < (uint32_t)L.nb[(size_t)l * N + c]) mask |= 0x11u << l;
+            }
+            own[c] = (uint8_t)mask;
+            n += (uint32_t)__builtin_popcount(mask & 0xFu);
+        }
         L.face_off[b + 1] = n;
     }
     for (uint32_t b = 0; b < nblk; ++b) L.face_off[b + 1] += L.face_off[b];
@@ -508,7 +509,7 @@ void build_faces(const Mesh& m, Layout& L) {
                 const uint32_t side = (inf >> 2) & 1u;
                 if (l == 0) L.cell_sum[c] = ((inf >> 8) & 0xFFu) | (((inf >> 16) & 0x7u) << dev::kSumCountShift);
                 L.cell_sum[c] |= (side << (dev::kSumSideShift + l)) | ((bnd ? 1u : 0u) << (dev::kSumBoundaryShift + l));
-                if (!lists(c, l)) continue;
+                if (!((own[c] >> l) & 1u)) continue;
                 const uint32_t other = (uint32_t)L.nb[o], nbs = inf & 3u;
                 const size_t e = (size_t)L.face_off[b] + n;
                 L.face_c0[e] = side ? other : c;
@@ -520,7 +521,7 @@ void build_faces(const Mesh& m, Layout& L) {
                 L.face_ny[e] = L.ny[o];
                 L.face_area[e] = L.area[o];
                 L.cell_faces[c] |= n << (8 * l);
-                if (shared(c, l)) L.cell_faces[other] |= n << (8 * nbs);
+                if ((own[c] >> (4 + l)) & 1u) L.cell_faces[other] |= n << (8 * nbs);
                 ++n;
             }
     }

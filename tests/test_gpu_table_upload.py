@@ -1,0 +1,24 @@
+"""A context's tables in one allocation (runs on an MI355X): sent in one copy up
+to 4 MiB (about 16,200 quads or 20,000 triangles), each in its own above.
+Residual parts on both sides of the line and on one cell, with fixed states
+among the boundaries, bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+from test_gpu_flux_blocks import BCS, random_state
+from test_gpu_parity import pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,nx,ny,recon", [("cartesian", 1, 1, "FO"), ("cartesian", 125, 125, "FO"),
+                                              ("cartesian", 131, 131, "FO"), ("cartesian_tri", 95, 95, "TENO"),
+                                              ("cartesian_tri", 107, 107, "TENO")])
+def test_residual(mlr, oracle, kind, nx, ny, recon):
+    kw = dict(recon=recon, riemann="Rusanov", bcs=BCS, p_ref=1.0, T_ref=1.0 / 287.0, rho_ref=1.0)
+    if recon == "TENO":
+        kw.update(order=2, teno_variant="corrected")
+    dev, orc, m = pair(mlr, oracle, kind, nx, ny, **kw)
+    U = random_state(m.n_cells, nx + ny)
+    for parts in (1, 2, 3):
+        assert np.array_equal(dev.calc_rhs_of(U, parts), orc.calc_rhs_parts(U, parts)), parts
