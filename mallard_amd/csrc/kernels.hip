@@ -1166,7 +1166,7 @@ __device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, co
     if (first >= N) return;  // whole block past the end (uniform)
     const uint32_t last = N - first < bs ? N : first + bs;
     const uint32_t f0 = g.face_off[first >> 6], nf = g.face_off[(last + 63u) >> 6] - f0;
-    __shared__ unsigned long long sh_max[JOIN ? 4 : 1];
+    __shared__ unsigned long long sh_max[JOIN ? 8 : 1];  // a wave each
     unsigned long long m = 0ull;
     auto share = [&]() {
         m = wave_max(m);
@@ -1228,7 +1228,7 @@ __device__ __forceinline__ void flux_block(const Geom& g, const StageArgs& a, co
 }
 
 template <int RS, bool PP, bool VISC, bool JOIN>
-__global__ __launch_bounds__(256) void flux_update_kernel(Geom g, StageArgs a, Physics ph, uint32_t bs,
+__global__ __launch_bounds__(512) void flux_update_kernel(Geom g, StageArgs a, Physics ph, uint32_t bs,
                                                           uint32_t blocks_per_xcd, DtJoin jn) {
     extern __shared__ __align__(16) unsigned char flux_smem[];
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
@@ -1787,8 +1787,14 @@ namespace {
 // triangles 8.9 us against 14.1 us with one thread per cell, 131,072
 // triangles 16.3 against 18.2. On larger meshes the second half of the block
 // idles in the cell sums: 2,097,152 triangles 174 us with one thread per
-// cell, 190 with two; they cross near 262,144 (30.6 us both).
-uint32_t flux_threads(uint32_t bs, uint64_t cells) { return bs < 256 && cells <= (1u << 18) ? 2 * bs : bs; }
+// cell, 190 with two; they cross near 262,144 (30.6 us both). Blocks of 256
+// cells, of which a CU holds half as many, cross between 131,072 and 245,000:
+// HLLC stage of 8,192 triangles 16.0 -> 13.6 us, 90,000 quads 22.9 -> 19.1,
+// Rusanov of 1,000 quads 11.6 -> 10.3; 245,000 triangles 27.2 -> 27.6, with
+// Roe 20.1 -> 21.4. An ensemble's blocks have at most 256 threads.
+uint32_t flux_threads(uint32_t bs, uint64_t cells) {
+    return cells <= (bs < 256 ? 1u << 18 : 1u << 17) ? 2 * bs : bs;
+}
 int face_size(uint32_t bs) { return bs == 64 ? 0 : (bs == 128 ? 1 : 2); }
 }  // namespace
 
@@ -1923,7 +1929,7 @@ hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_
                       const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
-    const dim3 grid(8 * per_xcd), block(flux_threads(bs, (uint64_t)total_blocks * bs));
+    const dim3 grid(8 * per_xcd), block(bs < 256 ? flux_threads(bs, (uint64_t)total_blocks * bs) : bs);
     const size_t lds = (size_t)face_max * 32;
 #define MLR_FBK(RSV, PPV)                                                                                       \
     do {                                                                                                        \

@@ -297,8 +297,8 @@ void Solver::setup(Mesh&& mesh) {
     HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     upload();
     // shapes of contexts that are not autotuned (programs that only call the
-    // residual): HLLC flux pass of 8,192 triangles 8.9 us with 128-cell
-    // blocks, 15.8 with 256; of 524,288 52 us with either; of 2,097,152 190
+    // residual): HLLC flux and update of 8,192 triangles 11.3 us with 128-cell
+    // blocks, 13.6 with 256; of 524,288 52 us with either; of 2,097,152 190
     // against 174. The derived face basis pays where the pass is bound by
     // bytes: 262,088 cells 4 us of 162, 8,388,608 cells 166 us of 4,671; below
     // it costs up to 1.6 us
@@ -1072,8 +1072,9 @@ void Solver::autotune() {
                    : cfg_.integrator == Integrator::RK4 ? dev::kRK4_1 : dev::kSSP1;
     // up to 262,144 cells 128-cell blocks, untimed: the flux kernel's length is
     // one thread's chain there, which the (often uniform) initial state does
-    // not show. A Sod step of 1,000 quads 36 us with 128, 42 with 64, 47 with
-    // 256; of 8,192 triangles 81, 81 and 102; of 102,659 quads 71, 74 and 75
+    // not show. An HLLC step of 1,000 quads 34 us with 128, 39 with 64 or 256;
+    // a TENO step of 8,192 triangles 51, 50 and 54; a Rusanov step of 102,659
+    // quads (RK4) 50, 54 and 51
     bt = 1e30f;
     best.flux_block = 128;
     for (uint32_t bs : {64u, 128u, 256u}) {
