@@ -194,8 +194,8 @@ void Ensemble::autotune() {
         upload_table();
         const float t = timed([&] {
             hip_ok(dev::spectral_batch(d_cases_, flux_case(), flux_blocks_, ph_, bs, stream_), "spectral_batch");
-            hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
-                   "flux_batch");
+            hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs),
+                                   stream_), "flux_batch");
         });
         if (t < bt) { bt = t; best.flux_block = bs; }
     }
@@ -220,8 +220,8 @@ void Ensemble::autotune() {
                 if (fb == 0 && (occ == 4 || (occ != 0 && !occ_tunable))) continue;
                 if (fb == 1 && occ == 6) continue;
                 const float t = timed([&] {
-                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
-                                           0, split_, fb == 1, ph_, stream_), "teno_batch");
+                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_,
+                                           gated_, occ, 0, split_, fb == 1, ph_, stream_), "teno_batch");
                 });
                 if (t < bt) { bt = t; best.teno_occ = occ; best.teno_face_basis = fb; }
             }
@@ -231,8 +231,8 @@ void Ensemble::autotune() {
             for (int occ : {0, 5, 6}) {
                 if (occ != 0 && !occ_tunable) continue;
                 const float t = timed([&] {
-                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_, gated_, occ,
-                                           1, split_, false, ph_, stream_), "teno_batch");
+                    hip_ok(dev::teno_batch(d_cases_, teno_case(), teno_blocks_, dev::kBufUn, K_, M_, FQ_, small_,
+                                           gated_, occ, 1, split_, false, ph_, stream_), "teno_batch");
                 });
                 if (t < bt) { bt = t; best.teno_occ_reuse = occ; }
             }
@@ -269,7 +269,8 @@ void Ensemble::launch_step(bool prof) {
     (void)prof;
     const int64_t cap = cases_[0]->dt_hist_cap_;
     const uint32_t bs = tune_.flux_block;
-    if (cfg_.use_cfl) hip_ok(dev::spectral_batch(d_cases_, flux_case(), flux_blocks_, ph_, bs, stream_), "spectral_batch");
+    if (cfg_.use_cfl)
+        hip_ok(dev::spectral_batch(d_cases_, flux_case(), flux_blocks_, ph_, bs, stream_), "spectral_batch");
     const double fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
     const bool join = joins();  // the first stage's flux pass finds the time steps
     if (!join)
@@ -293,8 +294,8 @@ void Ensemble::launch_step(bool prof) {
             st.fixed_dt = fixed_dt;
             st.hist_cap = cap;
         }
-        hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs), stream_),
-                   "flux_batch");
+        hip_ok(dev::flux_batch(d_cases_, flux_case(), flux_blocks_, st, (int)cfg_.riemann, ph_, bs, face_max(bs),
+                               stream_), "flux_batch");
         mark(kStatFluxMs);
     };
     if (cfg_.integrator == Integrator::SSPRK3) {
@@ -387,8 +388,9 @@ void Ensemble::launch_persistent(long long* clocks) {
     ps.cfl = cfg_.cfl;
     ps.fixed_dt = cfg_.use_cfl ? 0.0 : cfg_.dt;
     ps.hist_cap = cases_[0]->dt_hist_cap_;
-    hip_ok(dev::ensemble_step(d_cases_, size(), teno_case(), flux_case(), teno_blocks_, flux_blocks_, ps, (int)cfg_.riemann, teno_,
-                              face_max(256), ph_, stream_, &persistent_grid_), "ensemble_step");
+    hip_ok(dev::ensemble_step(d_cases_, size(), teno_case(), flux_case(), teno_blocks_, flux_blocks_, ps,
+                              (int)cfg_.riemann, teno_, face_max(256), ph_, stream_, &persistent_grid_),
+           "ensemble_step");
 }
 
 void Ensemble::finish(int64_t s0, int64_t n) {

@@ -281,7 +281,8 @@ __device__ __forceinline__ void teno_block(const Geom& g, const Teno& t, const d
         // every lane of a wave takes part in its loads, so a streamed pass
         // runs whole waves: those that hold a cell it reconstructs
         static_assert((GM == 0 || GM == 5) && MP > 0 && !CT, "streamed tables: a full pass at a compiled stencil size");
-        if (kFullOnly) streams = ((marks >> (8 * __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)))) & 0xFFu) != 0u;
+        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        if (kFullOnly) streams = ((marks >> (8 * w)) & 0xFFu) != 0u;
         if (streams) {
             stream.init(t, lb, sh_net);
 #pragma unroll
@@ -752,6 +753,8 @@ void teno_kernel(Geom g, Teno t, const double* __restrict__ U,
 // keeps the other blocks from being started: with a grid over every block
 // 64 us streamed and 34 not; at 8,388,608 cells 47 us against 123 for the
 // grid without streaming. Four members ahead and two blocks a CU: the same.
+// A list of every block costs: with no cell gated the three passes of a step
+// of 2,097,152 cells take 1,131 us each instead of 1,110.
 constexpr uint32_t kUngatedBlocks = 2048;  // two of the chip's fill; each walks its share of the list
 constexpr int kUngatedDepth = 2;
 template <bool CT>
@@ -817,8 +820,8 @@ void teno_stream_kernel(Geom g, Teno t, const double* __restrict__ U, double* __
                         uint8_t* __restrict__ dec, Physics ph, uint32_t tile_bytes, uint32_t blocks_per_xcd) {
     extern __shared__ __align__(16) unsigned char teno_smem[];
     const uint32_t lb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
-    teno_block<KP, MP, FQ, IdxT, 0, 0, false, false, SD>(g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem),
-                                                      teno_smem + tile_bytes);
+    teno_block<KP, MP, FQ, IdxT, 0, 0, false, false, SD>(
+        g, t, U, fs, dec, ph, lb, reinterpret_cast<double2*>(teno_smem), teno_smem + tile_bytes);
 }
 
 __device__ inline const double* case_buf(const CaseBufs& c, int role) {
@@ -1018,7 +1021,7 @@ __device__ inline void viscous_face(const Physics& ph, const Geom& g, const Stag
 // cells 22.8 -> 16 us. Holding the registers (about 100 for HLLC, 4 waves
 // per SIMD) to 5 waves costs time: 8,388,608 cells 957 us against 895, at 6
 // waves 1,110 us. So does pooling the faces that take the two-rarefaction
-// estimate, its powers more than half of a flux's instructions, onto the
+// estimate, its three powers 550 of a flux's 1,300 instructions, onto the
 // block's first threads through LDS: 524,288 cells 57.4 us against 50.1, the
 // two barriers and the 28 more registers cost more than the idle lanes.
 // RS: Riemann solver (compile-time, so each instantiation carries one
@@ -1146,10 +1149,12 @@ __device__ __forceinline__ void stage_update(const StageArgs& a, const Physics& 
 }
 
 // JOIN: the pass is a step's first and finds the time step. Every block joins
-// the block maxima of the radii (at most 4 a thread, loaded before the faces
-// and joined at the barrier after them), so the step has no launch of one
-// block for it: 4.5 us of 82 at 8,192 cells, while a block's join adds under
-// 1 us. Above kJoinBlocks maxima one block joins them in its own launch.
+// the block maxima of the radii (at most kJoinBlocks over its threads: 2 each
+// of 512 to 16 each of the 64 of a large ensemble's smallest blocks; loaded
+// before the faces and joined at the barrier after them), so the step has no
+// launch of one block for it: 4.5 us of 82 at 8,192 cells, while a block's join
+// adds under 1 us. Above kJoinBlocks maxima one block joins them in its own
+// launch.
 __device__ inline unsigned long long wave_max(unsigned long long m) {
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_xor(m, off);
@@ -1258,8 +1263,9 @@ __device__ inline StageArgs case_stage(const CaseBufs& cs, int op, int riemann, 
 // The flux + stage update of every case in one launch (blocks of bs cells;
 // the case table's block offsets count blocks of that size).
 template <int RS, bool PP, bool JOIN>
-__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __restrict__ flux_case,
-                                                         BatchStage st, uint32_t total, Physics ph, uint32_t bs,
+__global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restrict__ cases,
+                                                         const uint32_t* __restrict__ flux_case, BatchStage st,
+                                                         uint32_t total, Physics ph, uint32_t bs,
                                                          uint32_t blocks_per_xcd) {
     extern __shared__ __align__(16) unsigned char flux_smem[];
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
@@ -1267,7 +1273,8 @@ __global__ __launch_bounds__(256) void flux_batch_kernel(const CaseBufs* __restr
     const CaseBufs& cs = cases[flux_case[gb]];
     const StageArgs a = case_stage(cs, st.op, RS, st.fo, st.corrected, st.in, st.out);
     DtJoin jn{};
-    if constexpr (JOIN) jn = DtJoin{cs.lam_blk, (cs.g.N + bs - 1) / bs, st.cfl, st.fixed_dt, cs.dt, cs.dt_hist, st.hist_cap, cs.step};
+    if constexpr (JOIN)
+        jn = DtJoin{cs.lam_blk, (cs.g.N + bs - 1) / bs, st.cfl, st.fixed_dt, cs.dt, cs.dt_hist, st.hist_cap, cs.step};
     flux_block<RS, PP, false, JOIN>(cs.g, a, ph, gb - cs.blk_flux0, bs, reinterpret_cast<double*>(flux_smem), jn);
 }
 
@@ -1332,7 +1339,7 @@ __device__ __forceinline__ void spectral_block(const Geom& g, const double* __re
     if (threadIdx.x == 0) {
         unsigned long long m = sh[0];
         for (int i = 1; i < (int)(blockDim.x >> 6); ++i) m = sh[i] > m ? sh[i] : m;
-        lam_blk[lb] = m;  // the block's maximum; the finalize kernel joins the blocks
+        lam_blk[lb] = m;  // the block's maximum; the step's first flux pass or the finalize kernel joins them
     }
 }
 
@@ -1377,7 +1384,8 @@ __global__ __launch_bounds__(256) void spectral_kernel(Geom g, const double* __r
 
 // spectral radii of every case in one launch (each block inside one case, so
 // the block max goes to that case's maximum)
-__global__ __launch_bounds__(256) void spectral_batch_kernel(const CaseBufs* __restrict__ cases, const uint32_t* __restrict__ flux_case,
+__global__ __launch_bounds__(256) void spectral_batch_kernel(const CaseBufs* __restrict__ cases,
+                                                             const uint32_t* __restrict__ flux_case,
                                                              uint32_t total, Physics ph, uint32_t blocks_per_xcd) {
     const uint32_t gb = (blockIdx.x & 7u) * blocks_per_xcd + (blockIdx.x >> 3);
     if (gb >= total) return;
@@ -1462,9 +1470,10 @@ __device__ inline void grid_barrier(StepBarrier* bar, uint32_t n_blocks, long lo
 }
 
 template <int RS, bool TENO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void ensemble_step_kernel(const CaseBufs* __restrict__ cases, int n_cases, const uint32_t* __restrict__ teno_case, const uint32_t* __restrict__ flux_case,
-                                                            uint32_t teno_total, uint32_t flux_total,
-                                                            PersistentStep ps, Physics ph) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void ensemble_step_kernel(const CaseBufs* __restrict__ cases, int n_cases, const uint32_t* __restrict__ teno_case,
+                          const uint32_t* __restrict__ flux_case, uint32_t teno_total, uint32_t flux_total,
+                          PersistentStep ps, Physics ph) {
     extern __shared__ __align__(16) unsigned char step_smem[];
     const uint32_t G = gridDim.x, xcd = blockIdx.x & 7u, rank = blockIdx.x >> 3;
     const uint32_t on_xcd = (G + 7u - xcd) >> 3;
@@ -1646,10 +1655,11 @@ hipError_t teno_faces(const Geom& g, const Teno& t, const double* U, double* fs,
         if (!gate_reuse)
             if (const hipError_t e = list_mixed(t, g.N, stream); e != hipSuccess) return e;
         const dim3 ug(8 * per_xcd < kUngatedBlocks ? 8 * per_xcd : kUngatedBlocks);
+        const size_t tile = 256 * 32, slots = 4 * kUngatedDepth * (6 * 512 + 64);
         if (compact)
-            hipLaunchKernelGGL((teno_ungated_kernel<true>), ug, block, 256 * 32, stream, g, t, U, fs, dec, ph);
+            hipLaunchKernelGGL((teno_ungated_kernel<true>), ug, block, tile, stream, g, t, U, fs, dec, ph);
         else
-            hipLaunchKernelGGL((teno_ungated_kernel<false>), ug, block, 256 * 32 + 4 * kUngatedDepth * (6 * 512 + 64), stream, g, t, U, fs, dec, ph);
+            hipLaunchKernelGGL((teno_ungated_kernel<false>), ug, block, tile + slots, stream, g, t, U, fs, dec, ph);
         return hipGetLastError();
     };
     if (t.derived) {
@@ -1851,9 +1861,9 @@ hipError_t finalize_dt(const unsigned long long* lam_blk, uint32_t n_blk, double
     return hipGetLastError();
 }
 
-hipError_t teno_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, int in_role, int K, int M, int FQ,
-                      bool small, bool gated, int occ, int gate_reuse, bool split, bool derived, const Physics& ph,
-                      hipStream_t stream) {
+hipError_t teno_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, int in_role, int K,
+                      int M, int FQ, bool small, bool gated, int occ, int gate_reuse, bool split, bool derived,
+                      const Physics& ph, hipStream_t stream) {
     const int Kp = K - 1, Mp = M - 1;
     const size_t net_lds = (gated && !gate_reuse) ? ind::kNetInferBytes : 0;
     if ((FQ != 3 && FQ != 6) || Mp < 1) return hipErrorInvalidValue;
@@ -1925,20 +1935,20 @@ hipError_t teno_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_
     return hipGetLastError();
 }
 
-hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const BatchStage& st, int riemann,
-                      const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream) {
+hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const BatchStage& st,
+                      int riemann, const Physics& ph, uint32_t bs, uint32_t face_max, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
     const dim3 grid(8 * per_xcd), block(bs < 256 ? flux_threads(bs, (uint64_t)total_blocks * bs) : bs);
     const size_t lds = (size_t)face_max * 32;
-#define MLR_FBK(RSV, PPV)                                                                                       \
-    do {                                                                                                        \
-        if (st.join)                                                                                            \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, true>), grid, block, lds, stream, cases, block_case, st,  \
-                               total_blocks, ph, bs, per_xcd);                                                  \
-        else                                                                                                    \
-            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, false>), grid, block, lds, stream, cases, block_case, st, \
-                               total_blocks, ph, bs, per_xcd);                                                  \
+#define MLR_FBK(RSV, PPV)                                                                                           \
+    do {                                                                                                           \
+        if (st.join)                                                                                               \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, true>), grid, block, lds, stream, cases, block_case,   \
+                               st, total_blocks, ph, bs, per_xcd);                                                 \
+        else                                                                                                       \
+            hipLaunchKernelGGL((flux_batch_kernel<RSV, PPV, false>), grid, block, lds, stream, cases, block_case,  \
+                               st, total_blocks, ph, bs, per_xcd);                                                 \
     } while (0)
 #define MLR_FB(RSV)                      \
     do {                                 \
@@ -1957,8 +1967,8 @@ hipError_t flux_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_
     return hipGetLastError();
 }
 
-hipError_t spectral_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const Physics& ph, uint32_t bs,
-                          hipStream_t stream) {
+hipError_t spectral_batch(const CaseBufs* cases, const uint32_t* block_case, uint32_t total_blocks, const Physics& ph,
+                          uint32_t bs, hipStream_t stream) {
     if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
     const uint32_t per_xcd = (total_blocks + 7) / 8;
     hipLaunchKernelGGL(spectral_batch_kernel, dim3(8 * per_xcd), dim3(bs), 0, stream, cases, block_case, total_blocks,
@@ -2009,10 +2019,10 @@ hipError_t ensemble_step(const CaseBufs* cases, int n_cases, const uint32_t* ten
                          hipStream_t stream, int* grid_out) {
     if (n_cases < 1 || ps.n_stages < 1 || ps.n_stages > 4) return hipErrorInvalidValue;
 #define MLR_STEP(RSV)                                                                                          \
-    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_case, flux_case, teno_total, flux_total, ps, face_max, ph, stream, \
-                                                    grid_out)                                                    \
-                : launch_step_persistent<RSV, false>(cases, n_cases, teno_case, flux_case, teno_total, flux_total, ps, face_max, ph, stream, \
-                                                     grid_out)
+    return teno ? launch_step_persistent<RSV, true>(cases, n_cases, teno_case, flux_case, teno_total, flux_total, ps, \
+                                                    face_max, ph, stream, grid_out)                                 \
+                : launch_step_persistent<RSV, false>(cases, n_cases, teno_case, flux_case, teno_total, flux_total,  \
+                                                     ps, face_max, ph, stream, grid_out)
     switch (riemann) {
     case 0: MLR_STEP(0);
     case 1: MLR_STEP(1);

@@ -442,8 +442,8 @@ void teno_matrices_of_cell(const Mesh& m, const TenoSpec& ts, uint32_t c,
 uint64_t Layout::device_bytes() const {
     auto b = [](const auto& v) { return (uint64_t)v.size() * sizeof(v[0]); };
     return b(volume) + b(nb) + b(info) + b(nx) + b(ny) + b(area) + b(dxn) + b(face_off) + b(face_c0) + b(face_c1) +
-           b(face_meta) + b(face_nx) + b(face_ny) + b(face_area) + b(cell_faces) + b(cell_sum) + b(blk_off) + b(blk_ids) +
-           b(st_loc8) + b(st_loc16) + b(st_ta) +
+           b(face_meta) + b(face_nx) + b(face_ny) + b(face_area) + b(cell_faces) + b(cell_sum) + b(blk_off) +
+           b(blk_ids) + b(st_loc8) + b(st_loc16) + b(st_ta) +
            b(st_A) + b(fbasis);
 }
 

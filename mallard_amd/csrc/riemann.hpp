@@ -28,11 +28,11 @@ __device__ inline void prims(const Physics& ph, const double* U, double* W) {
 }
 
 // ------------------------------------------------------------ Riemann
-// Quotients of the specific-heat ratio come with the gas, and the powers of
-// the two-rarefaction estimate, a third of an HLLC flux's instructions, take
-// their table index from one FP32 logarithm and share a reciprocal between
-// their two quotients: flux pass of 8,388,608 cells 973 -> 871 us, 524,288
-// 53.1 -> 49.5, 8,192 10.3 -> 8.5.
+// Quotients of the specific-heat ratio come with the gas, and the three powers
+// of the two-rarefaction estimate (about 180 vector instructions each, in a
+// flux of about 1,300) take their table index from one FP32 logarithm and
+// share a reciprocal between their two quotients: flux pass of 8,388,608 cells
+// 973 -> 871 us, 524,288 53.1 -> 49.5, 8,192 10.3 -> 8.5.
 // riemann_solver.h:205-240
 __device__ inline void pvrs(const double* Wl, const double* Wr, double& ps) {
     const double rl = Wl[0], ul = Wl[1], pl = Wl[2], gl = Wl[3];

@@ -1187,7 +1187,7 @@ void Solver::finish_steps(int64_t s0, int64_t n, double* dts_out) {
 void Solver::set_dt_history(int64_t cap) {
     if (cap < 1 || cap > kDtHistCap) fail("the dt history holds 1 to 1048576 steps");
     synchronize();
-    drop_graph();  // the captured finalize kernel carries the ring's address and length
+    drop_graph();  // the captured flux pass (or finalize kernel) carries the ring's address and length
     void* p = nullptr;
     HIP_OK(hipMalloc(&p, sizeof(double) * cap));
     HIP_OK(hipMemset(p, 0, sizeof(double) * cap));

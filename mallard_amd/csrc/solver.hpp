@@ -237,7 +237,8 @@ private:
     uint32_t* info_ = nullptr;
     uint32_t* perm_ = nullptr;  // reference row of each cell
     // face lists of the flux kernel
-    uint32_t *face_off_ = nullptr, *face_c0_ = nullptr, *face_c1_ = nullptr, *cell_faces_ = nullptr, *cell_sum_ = nullptr;
+    uint32_t *face_off_ = nullptr, *face_c0_ = nullptr, *face_c1_ = nullptr;
+    uint32_t *cell_faces_ = nullptr, *cell_sum_ = nullptr;
     uint16_t* face_meta_ = nullptr;
     double *face_nx_ = nullptr, *face_ny_ = nullptr, *face_area_ = nullptr;
     dev::BCParam* bc_ = nullptr;

@@ -44,7 +44,8 @@ extern "C" long check_face_lists(uint32_t n_nodes, const double* xy, uint32_t n_
             if (ok) {
                 const uint32_t meta = L.face_meta[e], s0 = meta & 3u, s1 = (meta >> dev::kFaceSlot1Shift) & 3u;
                 ok = L.face_c0[e] == (side ? nb : c) && L.face_c1[e] == (side ? c : nb) &&
-                     ((meta & dev::kFaceBoundary) != 0) == bnd && s0 == (side ? nbs : l) && (bnd || s1 == (side ? l : nbs)) &&
+                     ((meta & dev::kFaceBoundary) != 0) == bnd &&
+                     s0 == (side ? nbs : l) && (bnd || s1 == (side ? l : nbs)) &&
                      L.face_nx[e] == L.nx[o] && L.face_ny[e] == L.ny[o] && L.face_area[e] == L.area[o];
             }
             bad += ok ? 0 : 1;
