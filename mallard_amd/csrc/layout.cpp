@@ -465,7 +465,7 @@ void build_faces(const Mesh& m, Layout& L) {
     // per cell: bit l where slot l lists its face (it contributes to the
     // residual, and no lower cell of the block lists it), bit 4 + l where the
     // entry serves the neighbour too
-    std::vector<uint8_t> own(N);
+    Table<uint8_t> own(N);
     L.face_off.assign(nblk + 1, 0);
 #pragma omp parallel for schedule(static)
     for (int64_t b = 0; b < (int64_t)nblk; ++b) {
@@ -495,11 +495,12 @@ void build_faces(const Mesh& m, Layout& L) {
     L.face_nx.resize(nf);
     L.face_ny.resize(nf);
     L.face_area.resize(nf);
-    L.cell_faces.assign(N, 0);
-    L.cell_sum.assign(N, 0);
+    L.cell_faces.resize(N);
+    L.cell_sum.resize(N);
 #pragma omp parallel for schedule(static)
     for (int64_t b = 0; b < (int64_t)nblk; ++b) {
         const uint32_t c0 = (uint32_t)b * B, c1 = std::min(N, c0 + B);
+        std::fill(&L.cell_faces[c0], &L.cell_faces[c0] + (c1 - c0), 0u);
         uint32_t n = 0;  // at most 64 S <= 256 entries: 8-bit positions
         for (uint32_t l = 0; l < S; ++l)
             for (uint32_t c = c0; c < c1; ++c) {
@@ -617,16 +618,9 @@ Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::v
     const uint32_t S = L.S;
     L.volume.resize(N);
     L.centroid.resize(2 * (size_t)N);
-    L.nb.assign((size_t)S * N, 0);
-    L.info.assign((size_t)S * N, 0);
-    L.nx.assign((size_t)S * N, 0.0);
-    L.ny.assign((size_t)S * N, 0.0);
-    L.area.assign((size_t)S * N, 0.0);
-    L.dxn.assign((size_t)S * N, 0.0);
-    L.dcx.assign((size_t)S * N, 0.0);
-    L.dcy.assign((size_t)S * N, 0.0);
-    L.mfx.assign((size_t)S * N, 0.0);
-    L.mfy.assign((size_t)S * N, 0.0);
+    L.nb.resize((size_t)S * N);
+    L.info.resize((size_t)S * N);
+    for (auto* v : {&L.nx, &L.ny, &L.area, &L.dxn, &L.dcx, &L.dcy, &L.mfx, &L.mfy}) v->resize((size_t)S * N);
     L.face_slot.assign(m.n_faces, ~0u);
     bool bad = false;
 #pragma omp parallel for schedule(static)

@@ -6,7 +6,10 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "common.hpp"
@@ -47,6 +50,26 @@ struct TenoSpec {
 constexpr uint32_t kSlotBoundary = 1u << 3;
 constexpr uint32_t kNoBC = 15u;
 
+// Allocator of tables that a parallel loop writes whole: their memory is not
+// cleared first, so each thread is the first to touch its part.
+template <class T>
+struct Uncleared : std::allocator<T> {
+    template <class U>
+    struct rebind {
+        using other = Uncleared<U>;
+    };
+    template <class U>
+    void construct(U* p) noexcept {
+        ::new (static_cast<void*>(p)) U;
+    }
+    template <class U, class... Args>
+    void construct(U* p, Args&&... args) {
+        ::new (static_cast<void*>(p)) U(std::forward<Args>(args)...);
+    }
+};
+template <class T>
+using Table = std::vector<T, Uncleared<T>>;
+
 struct Layout {
     uint32_t N = 0;        // cells
     uint32_t S = 0;        // face slots per cell (3 triangles, 4 quads)
@@ -57,13 +80,13 @@ struct Layout {
     std::vector<uint32_t> iperm;  // old -> new
     std::vector<uint32_t> face_slot;  // old face id -> (new cell << 2 | slot) of side 0, or ~0u
 
-    std::vector<double> volume;           // [N]
-    std::vector<double> centroid;         // [N][2] (new numbering, for init/output)
-    std::vector<int32_t> nb;              // [S][N] neighbour (new id), self for boundary slots
-    std::vector<uint32_t> info;           // [S][N]
-    std::vector<double> nx, ny, area, dxn;  // [S][N]
-    std::vector<double> dcx, dcy;           // [S][N] centroid to neighbour centroid (face midpoint on boundaries)
-    std::vector<double> mfx, mfy;           // [S][N] centroid to face midpoint
+    Table<double> volume;           // [N]
+    Table<double> centroid;         // [N][2] (new numbering, for init/output)
+    Table<int32_t> nb;              // [S][N] neighbour (new id), self for boundary slots
+    Table<uint32_t> info;           // [S][N]
+    Table<double> nx, ny, area, dxn;  // [S][N]
+    Table<double> dcx, dcy;           // [S][N] centroid to neighbour centroid (face midpoint on boundaries)
+    Table<double> mfx, mfy;           // [S][N] centroid to face midpoint
 
     // Face lists of the flux kernel: block b = cells [64b, 64b+64). Entries
     // face_off[b] .. face_off[b+1] hold every face of the block's cells that
@@ -71,11 +94,11 @@ struct Layout {
     // face between two blocks one entry in each. Ordered by the slot and the
     // cell that lists the face (the lower cell of a face inside the block).
     std::vector<uint32_t> face_off;         // [n_blocks + 1]
-    std::vector<uint32_t> face_c0, face_c1; // side-0 and side-1 cell (side 0 again on boundaries)
-    std::vector<uint16_t> face_meta;        // dev::kFace* bits
-    std::vector<double> face_nx, face_ny, face_area;
-    std::vector<uint32_t> cell_faces;       // [N] in-block entry of each slot's face, 8 bits per slot
-    std::vector<uint32_t> cell_sum;         // [N] dev::kSum* bits: order, count and signs of the face sum
+    Table<uint32_t> face_c0, face_c1;       // side-0 and side-1 cell (side 0 again on boundaries)
+    Table<uint16_t> face_meta;              // dev::kFace* bits
+    Table<double> face_nx, face_ny, face_area;
+    Table<uint32_t> cell_faces;             // [N] in-block entry of each slot's face, 8 bits per slot
+    Table<uint32_t> cell_sum;               // [N] dev::kSum* bits: order, count and signs of the face sum
     uint32_t face_max[3] = {0, 0, 0};       // most entries of 1, 2 and 4 consecutive blocks (from a multiple of it)
 
     // TENO (empty for FO): G = S + 1 stencils per cell, K = n_dof, M = cells per stencil.

@@ -372,10 +372,11 @@ void Solver::upload() {
     const size_t N = L_.N;
     // The tables of every run in one allocation, each from a multiple of 256
     // bytes on; up to kStaged bytes they go over in one copy. Building a
-    // context of 1,000 quads takes 402 us, with an allocation and a copy per
-    // table 642; 40,000 quads 6.0 ms and 6.4. Above, the staging would copy
-    // every table once more on the host for nothing that counts.
-    constexpr size_t kStaged = 4u << 20;
+    // context of 1,000 quads took 642 us with an allocation and a copy per
+    // table, 402 so, one of 25,600 (6.6 MB) 3.2 ms and 2.6. Above, touching the
+    // staging memory costs more than the copies: 63,000 quads (16 MB) staged
+    // 12.0 ms, not staged 9.0.
+    constexpr size_t kStaged = 8u << 20;
     struct Table {
         void** dst;
         const void* src;

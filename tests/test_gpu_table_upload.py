@@ -1,5 +1,5 @@
 """A context's tables in one allocation (runs on an MI355X): sent in one copy up
-to 4 MiB (about 16,200 quads or 20,000 triangles), each in its own above.
+to 8 MiB (about 32,700 quads or 42,300 triangles), each in its own above.
 Residual parts on both sides of the line and on one cell, with fixed states
 among the boundaries, bit for bit against the oracle."""
 import numpy as np
@@ -11,9 +11,9 @@ from test_gpu_parity import pair
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind,nx,ny,recon", [("cartesian", 1, 1, "FO"), ("cartesian", 125, 125, "FO"),
-                                              ("cartesian", 131, 131, "FO"), ("cartesian_tri", 95, 95, "TENO"),
-                                              ("cartesian_tri", 107, 107, "TENO")])
+@pytest.mark.parametrize("kind,nx,ny,recon", [("cartesian", 1, 1, "FO"), ("cartesian", 178, 180, "FO"),
+                                              ("cartesian", 183, 181, "FO"), ("cartesian_tri", 143, 145, "TENO"),
+                                              ("cartesian_tri", 149, 147, "TENO")])
 def test_residual(mlr, oracle, kind, nx, ny, recon):
     kw = dict(recon=recon, riemann="Rusanov", bcs=BCS, p_ref=1.0, T_ref=1.0 / 287.0, rho_ref=1.0)
     if recon == "TENO":
