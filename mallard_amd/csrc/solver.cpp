@@ -1011,9 +1011,13 @@ void Solver::autotune() {
     dev::Tune best = tune_;
     const bool prof = prof_on_;
     prof_on_ = false;
-    // spectral radius block
+    // spectral radius block: of those that leave few enough maxima for the
+    // step's first flux pass to join, where one does. The kernel alone differs
+    // by parts of a microsecond between them; the join's own launch costs 3.3 us
+    // a step (73,006 cells, 64-cell blocks against 128)
     float bt = 1e30f;
     for (uint32_t bs : {64u, 128u, 256u}) {
+        if ((L_.N + bs - 1) / bs > dev::kJoinBlocks && (L_.N + 255) / 256 <= dev::kJoinBlocks) continue;
         const float t = timed([&] {
             HIP_OK(dev::spectral_radius(geom(), Un_, prims_, ph_, lam_cell_, lam_blk_, bs, stream_));
         });
