@@ -578,7 +578,7 @@ void build_tiles(Layout& L) {
 }
 
 Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::vector<BoundarySpec>& bcs,
-                    int n_threads, bool allow_device) {
+                    int n_threads, bool allow_device, bool viscous) {
 #ifdef _OPENMP
     if (n_threads > 0) omp_set_num_threads(n_threads);
 #endif
@@ -620,7 +620,9 @@ Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::v
     L.centroid.resize(2 * (size_t)N);
     L.nb.resize((size_t)S * N);
     L.info.resize((size_t)S * N);
-    for (auto* v : {&L.nx, &L.ny, &L.area, &L.dxn, &L.dcx, &L.dcy, &L.mfx, &L.mfy}) v->resize((size_t)S * N);
+    for (auto* v : {&L.nx, &L.ny, &L.area, &L.dxn}) v->resize((size_t)S * N);
+    if (viscous)
+        for (auto* v : {&L.dcx, &L.dcy, &L.mfx, &L.mfy}) v->resize((size_t)S * N);
     L.face_slot.assign(m.n_faces, ~0u);
     bool bad = false;
 #pragma omp parallel for schedule(static)
@@ -670,17 +672,12 @@ Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts, const std::v
             L.dxn[o] = std::fabs(s0 * u0 + s1 * u1);
             // viscous face gradients: the vector the directional correction
             // runs along, and the one to the face midpoint
-            {
+            if (viscous) {
                 const uint32_t a = m.node_of_face(f, 0), b = m.node_of_face(f, 1);
                 L.mfx[o] = 0.5 * (m.nc(a, 0) + m.nc(b, 0)) - m.cc(c, 0);
                 L.mfy[o] = 0.5 * (m.nc(a, 1) + m.nc(b, 1)) - m.cc(c, 1);
-            }
-            if (bnd) {
-                L.dcx[o] = L.mfx[o];
-                L.dcy[o] = L.mfy[o];
-            } else {
-                L.dcx[o] = m.cc(other, 0) - m.cc(c, 0);
-                L.dcy[o] = m.cc(other, 1) - m.cc(c, 1);
+                L.dcx[o] = bnd ? L.mfx[o] : m.cc(other, 0) - m.cc(c, 0);
+                L.dcy[o] = bnd ? L.mfy[o] : m.cc(other, 1) - m.cc(c, 1);
             }
             keys[l] = key[f];
         }

@@ -85,6 +85,7 @@ struct Layout {
     Table<int32_t> nb;              // [S][N] neighbour (new id), self for boundary slots
     Table<uint32_t> info;           // [S][N]
     Table<double> nx, ny, area, dxn;  // [S][N]
+    // viscous layouts only
     Table<double> dcx, dcy;           // [S][N] centroid to neighbour centroid (face midpoint on boundaries)
     Table<double> mfx, mfy;           // [S][N] centroid to face midpoint
 
@@ -158,8 +159,10 @@ std::vector<uint32_t> sfc_order(const Mesh& m);
 // Builds the layout. bcs lists the boundary conditions in input order.
 // allow_device: leave the pseudo-inverses to the GPU precompute when it
 // supports the basis and stencil size (the host still searches stencils).
+// viscous: with the vectors of the viscous face gradients (dcx, dcy, mfx, mfy).
 Layout build_layout(const Mesh& m, Recon recon, const TenoSpec& ts,
-                    const std::vector<BoundarySpec>& bcs, int n_threads = 0, bool allow_device = false);
+                    const std::vector<BoundarySpec>& bcs, int n_threads = 0, bool allow_device = false,
+                    bool viscous = false);
 
 // Reference-numbered stencil lists recomputed for one cell (used by the
 // index-parity tests through the C-ABI): out = G stencils of M ids each (or

@@ -293,7 +293,7 @@ void Solver::setup(Mesh&& mesh) {
     if (cfg_.positivity && cfg_.integrator == Integrator::RK4)
         fail("the positivity limiter needs forward Euler or SSP-RK3 (RK4 is no convex combination of Euler steps)");
     if (cfg_.positivity && cfg_.viscous) fail("the positivity limiter is for the Euler equations");
-    L_ = build_layout(mesh_, cfg_.recon, cfg_.teno, cfg_.bcs, cfg_.n_threads, /*allow_device=*/true);
+    L_ = build_layout(mesh_, cfg_.recon, cfg_.teno, cfg_.bcs, cfg_.n_threads, /*allow_device=*/true, cfg_.viscous);
     HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     upload();
     // shapes of contexts that are not autotuned (programs that only call the
@@ -377,12 +377,12 @@ void Solver::upload() {
     // staging memory costs more than the copies: 63,000 quads (16 MB) staged
     // 12.0 ms, not staged 9.0.
     constexpr size_t kStaged = 8u << 20;
-    struct Table {
+    struct Upload {
         void** dst;
         const void* src;
         size_t at, bytes;
     };
-    std::vector<Table> tables;
+    std::vector<Upload> tables;
     size_t total = 0;
     auto table = [&](auto*& dst, const auto& v) {
         const size_t bytes = v.size() * sizeof(v[0]);
@@ -436,14 +436,14 @@ void Solver::upload() {
         table(oi_, oi);
     }
     unsigned char* block = static_cast<unsigned char*>(dalloc(total));
-    for (const Table& t : tables) *t.dst = block + t.at;
+    for (const Upload& t : tables) *t.dst = block + t.at;
     if (total <= kStaged) {
         std::vector<unsigned char> staged(total);
-        for (const Table& t : tables)
+        for (const Upload& t : tables)
             if (t.bytes) std::memcpy(staged.data() + t.at, t.src, t.bytes);
         HIP_OK(hipMemcpy(block, staged.data(), total, hipMemcpyHostToDevice));
     } else {
-        for (const Table& t : tables)
+        for (const Upload& t : tables)
             if (t.bytes) HIP_OK(hipMemcpy(*t.dst, t.src, t.bytes, hipMemcpyHostToDevice));
     }
     if (L_.teno) {
@@ -484,6 +484,13 @@ void Solver::upload() {
         std::vector<double>().swap(L_.st_A);
         std::vector<double>().swap(L_.fbasis);
     }
+    // nor those of the geometry and the face lists
+    for (auto* v : {&L_.nx, &L_.ny, &L_.area, &L_.dxn, &L_.dcx, &L_.dcy, &L_.mfx, &L_.mfy, &L_.face_nx, &L_.face_ny,
+                    &L_.face_area})
+        Table<double>().swap(*v);
+    for (auto* v : {&L_.face_c0, &L_.face_c1, &L_.cell_faces, &L_.cell_sum}) Table<uint32_t>().swap(*v);
+    Table<uint16_t>().swap(L_.face_meta);
+    Table<int32_t>().swap(L_.nb);
     auto dz = [&](size_t n) {
         double* p = (double*)dalloc(n * sizeof(double));
         HIP_OK(hipMemset(p, 0, n * sizeof(double)));
